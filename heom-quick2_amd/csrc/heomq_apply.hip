@@ -4,15 +4,22 @@
 // BiCG convention).
 //
 // Mapping: the d*d elements of one output ADO are spread over min(d*d, 256)
-// lanes of a 256-thread workgroup (d = 4: 16 lanes per ADO, four ADOs per
-// wave64; d = 16: one ADO per workgroup; d = 64: 16 elements per lane).
-// Element (i, j) lives at complex offset i + j*d (the reference's Fortran
-// order), so consecutive lanes read consecutive rows: a column of a neighbour
-// block is one coalesced segment.  The ADO's own block is staged in LDS for
-// the H commutator; neighbour blocks are gathered straight from HBM/L2, one
-// element per lane per term, because c and c^+ are signed partial
-// permutations: (c X)(i, j) = s_i * X(p_i, j).
+// lanes of a 256-thread workgroup.  Element (i, j) lives at complex offset
+// i + j*d (the reference's Fortran order), so consecutive lanes read
+// consecutive rows: a column of a neighbour block is one coalesced segment.
+// The ADO's own block is staged in LDS for the H commutator; neighbour blocks
+// are gathered straight from HBM/L2, one element per lane per term, because c
+// and c^+ are signed partial permutations: (c X)(i, j) = s_i * X(p_i, j).
+//
+// An ADO below the top tier has one coupling per drawer (72 to 112), a
+// top-tier ADO one per drawer it holds (2 to 4), so the two run apart:
+// "heavy" workgroups take one ADO each, its couplings staged in LDS and
+// sliced over the lanes (256 / (d*d) slices at d = 4, one at d = 16), four
+// gathered at a time; "light" workgroups take 256 / (d*d) top-tier ADOs at a
+// time and a run of such groups, so the operator maps and H are staged once.
 #include "heomq_kernels.hpp"
+
+#include <algorithm>
 
 namespace heomq {
 
@@ -21,135 +28,275 @@ template <> struct V2<double> { using type = double2; };
 template <> struct V2<float> { using type = float2; };
 
 constexpr int kMaxOps = 12;   // 2 * norbs * nspin for norbs <= 3
+constexpr int kStage = 128;   // couplings staged in LDS at once
 
+// One coupling with its record: coefficients with the entry's signs, the
+// neighbour, the operator (0xff: no term) and the dagger flag.
+template <typename T>
+struct Coupling {
+  T clr, cli, crr, cri;
+  int32_t nbr;
+  uint8_t op, dag;
+};
+
+template <typename T>
+__device__ inline Coupling<T> to_coupling(const DevOperator& op, const DevEntry en) {
+  const double2* r = reinterpret_cast<const double2*>(op.rec + en.rec);
+  const double2 l = r[0], q = r[1];
+  const T sl = (en.flags & 2) ? (T)-1 : (T)1, sr = (en.flags & 4) ? (T)-1 : (T)1;
+  return Coupling<T>{sl * (T)l.x, sl * (T)l.y, sr * (T)q.x, sr * (T)q.y, en.nbr, en.op, (uint8_t)(en.flags & 1)};
+}
+
+// Couplings cs[0], cs[stride], .. (nv of them, at most U) of element (i, j):
+// every neighbour element is loaded before any is used.  smap[o * 2 * D + i] = (p_i + 1) * s_i of the left factor,
+// smap[o * 2 * D + D + j] the same of the right factor, 0 for no term.
+template <int D, typename T, bool TRANS, int U>
+__device__ inline void add_couplings(const Coupling<T>* cs, int stride, int nv, const int8_t* smap,
+                                     const typename V2<T>::type* __restrict__ xv, int i, int j, int64_t trace_pos,
+                                     int trace_elem, T& ar, T& ai) {
+  using V = typename V2<T>::type;
+  V vl[U], vr[U];
+  int ml[U], mr[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    vl[u] = V{0, 0};
+    vr[u] = V{0, 0};
+    ml[u] = mr[u] = 0;
+    if (u >= nv) continue;
+    const Coupling<T>& c = cs[u * stride];
+    if (c.op == 0xff) continue;
+    ml[u] = smap[c.op * 2 * D + i];
+    mr[u] = smap[c.op * 2 * D + D + j];
+    const V* __restrict__ xn = xv + (int64_t)c.nbr * (D * D);
+    const int pl = (ml[u] < 0 ? -ml[u] : ml[u]) - 1, pr = (mr[u] < 0 ? -mr[u] : mr[u]) - 1;
+    const int el = c.dag ? j + pl * D : pl + j * D, er = c.dag ? pr + i * D : i + pr * D;
+    if (ml[u] != 0 && !(TRANS && c.nbr == trace_pos && el == trace_elem)) vl[u] = xn[el];
+    if (mr[u] != 0 && !(TRANS && c.nbr == trace_pos && er == trace_elem)) vr[u] = xn[er];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u >= nv) break;
+    __builtin_amdgcn_sched_barrier(0);   // one coupling's coefficients in registers at a time
+    const Coupling<T>& c = cs[u * stride];
+    const T cj = c.dag ? (T)-1 : (T)1;
+    const T sl = ml[u] < 0 ? (T)-1 : (T)1, sr = mr[u] < 0 ? (T)-1 : (T)1;   // a zero element where there is no term
+    const T lx = sl * vl[u].x, ly = sl * cj * vl[u].y, rx = sr * vr[u].x, ry = sr * cj * vr[u].y;
+    ar += c.clr * lx - c.cli * ly;
+    ai += c.clr * ly + c.cli * lx;
+    ar += c.crr * rx - c.cri * ry;
+    ai += c.crr * ry + c.cri * rx;
+  }
+}
+
+// What a workgroup stages once: the operators' maps and, for d <= 16, H by
+// rows with the row index fastest (16 rows of one column index are
+// consecutive: no bank conflicts).
+template <int D>
+struct DenseLds {
+  static constexpr bool kH = D <= 16;
+  int8_t smap[kMaxOps * 2 * D];
+  uint8_t hn[kH ? D : 1];
+  uint8_t hc[kH ? D * D : 1];
+  double2 hv[kH ? D * D : 1];
+  __device__ void stage(const DevOperator& op) {
+    for (int k = threadIdx.x; k < op.nop * 2 * D; k += 256) {
+      const int o = k / (2 * D), r = k % (2 * D), side = r / D, i = r % D;
+      const int8_t* m = op.opmap + (o * 4 + 2 * side) * D;
+      smap[k] = m[i] < 0 ? (int8_t)0 : (int8_t)((m[i] + 1) * m[D + i]);
+    }
+    if (kH) {
+      if (threadIdx.x < D) hn[threadIdx.x] = (uint8_t)op.hnnz[threadIdx.x];
+      for (int k = threadIdx.x; k < D * D; k += 256) {
+        const int i = k % D, t = k / D;
+        if (t >= op.hnnz[i]) continue;
+        hc[k] = (uint8_t)op.hcol[i * D + t];
+        hv[k] = reinterpret_cast<const double2*>(op.hval)[i * D + t];
+      }
+    }
+  }
+  // i hsign (H X - X H)(i, j) + gamma X(i, j) of the block `self` (LDS)
+  template <typename T>
+  __device__ void same_tier(const DevOperator& op, const typename V2<T>::type* self, T gr, T gi, int i, int j, T& ar,
+                            T& ai) const {
+    using V = typename V2<T>::type;
+    const V xe = self[i + j * D];
+    T cr = 0, ci = 0;
+    const int ni = kH ? (int)hn[i] : op.hnnz[i];
+#pragma unroll 1
+    for (int t = 0; t < ni; ++t) {            // (H X)(i, j)
+      const int c = kH ? (int)hc[t * D + i] : op.hcol[i * D + t];
+      const double2 h = kH ? hv[t * D + i] : reinterpret_cast<const double2*>(op.hval)[i * D + t];
+      const V v = self[c + j * D];
+      cr += (T)h.x * v.x - (T)h.y * v.y;
+      ci += (T)h.x * v.y + (T)h.y * v.x;
+    }
+    const int nj = kH ? (int)hn[j] : op.hnnz[j];
+#pragma unroll 1
+    for (int t = 0; t < nj; ++t) {            // (X H)(i, j) = sum_k X(i, k) conj(H(j, k))
+      const int c = kH ? (int)hc[t * D + j] : op.hcol[j * D + t];
+      const double2 h = kH ? hv[t * D + j] : reinterpret_cast<const double2*>(op.hval)[j * D + t];
+      const V v = self[i + c * D];
+      cr -= (T)h.x * v.x + (T)h.y * v.y;
+      ci -= (T)h.x * v.y - (T)h.y * v.x;
+    }
+    const T hs = (T)op.hsign;
+    ar += gr * xe.x - gi * xe.y - hs * ci;
+    ai += gr * xe.y + gi * xe.x + hs * cr;
+  }
+};
+
+template <typename T>
+__device__ inline int tier_parity(const DevOperator& op, int64_t a) {
+  int n = 0;
+  while (n + 1 < op.tb.ntier && op.tb.first[n + 1] <= a) ++n;
+  return n & 1;
+}
+
+// Blocks [0, n_heavy) take one ADO below the top tier each; the rest take
+// `run` groups of 256 / min(d*d, 256) consecutive top-tier ADOs.
+//
+// Bound by the latency of the dependent loads (entry -> record -> neighbour
+// element) and, at d = 16, by HBM and the Infinity Cache: every top-tier block
+// is read by its own workgroup and by the three heavy ADOs above it.  Staging
+// the couplings in LDS takes entry and record out of the element's chain, and
+// the couplings in flight (4 heavy and 3 light at d = 16, 2 and 2 at d = 4)
+// are the most that keep 80 VGPRs without scratch, 6 waves per SIMD.  FP64
+// forward, with one ADO per workgroup slot and its couplings walked one by one
+// before: 1415 -> 514 us at two-impurity size (M = 112, L = 3; 962 MB, 1.9
+// TB/s), 71 -> 15 us and 441 -> 216 us at the single impurity's M = 72, L = 3
+// and 4.  Ordering the heavy workgroups among the light ones by their
+// neighbours' place gave 597 against 622 us at an earlier stage, for a table
+// built per context: not kept.
 template <int D, typename T, bool TRANS>
-__global__ void __launch_bounds__(256)
-k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_t trace_pos, int project) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 16 ? 6 : 2)))
+k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_t trace_pos, int project,
+        int64_t n_heavy, int run, int light_max) {
   using V = typename V2<T>::type;
   constexpr int E = D * D;
   constexpr int LANES = E < 256 ? E : 256;
   constexpr int EPT = E / LANES;
-  constexpr int APB = 256 / LANES;
-  __shared__ V xs[APB * E];
-  __shared__ int8_t sop[kMaxOps * 4 * D];
-
+  constexpr int APB = 256 / LANES;   // ADOs of a light group, slices of a heavy ADO
+  constexpr int U = EPT > 1 ? 1 : (D == 4 ? 2 : 4), UL = EPT > 1 ? 1 : (D == 4 ? 2 : 3);   // couplings in flight, heavy and light
+  __shared__ V xs[EPT == 1 ? 512 : E];
+  __shared__ DenseLds<D> tab;
+  __shared__ Coupling<T> s_c[kStage];
   const int tid = threadIdx.x;
-  for (int t = tid; t < op.nop * 4 * D; t += 256) sop[t] = op.opmap[t];
-  const int slot = tid / LANES;
-  const int lane = tid - slot * LANES;
-  const int64_t a = (int64_t)blockIdx.x * APB + slot;
-  const bool active = a < op.n_ado;
+  const int slot = APB > 1 ? tid / LANES : 0, lane = tid - slot * LANES;   // one ADO per group: uniform addresses
   const V* __restrict__ xv = reinterpret_cast<const V*>(x);
-  if (active) {
-#pragma unroll
-    for (int k = 0; k < EPT; ++k) {
-      const int e = lane + k * LANES;
-      V v = xv[a * E + e];
-      if (TRANS && a == trace_pos && e == op.trace_elem) { v.x = 0; v.y = 0; }
-      xs[slot * E + e] = v;
-    }
-  }
-  __syncthreads();
-  if (!active) return;   // no barrier follows
-  const V* self = &xs[slot * E];
-
-  T ar[EPT], ai[EPT];
-  const T gr = (T)op.gam[2 * a], gi = (T)op.gam[2 * a + 1];
-  const T hs = (T)op.hsign;
-#pragma unroll
-  for (int k = 0; k < EPT; ++k) {
-    const int e = lane + k * LANES;
-    const int i = e % D, j = e / D;
-    const V xe = self[e];
-    T cr = 0, ci = 0;
-    const int ni = op.hnnz[i];
-    for (int t = 0; t < ni; ++t) {            // (H X)(i, j)
-      const int c = op.hcol[i * D + t];
-      const T hr = (T)op.hval[2 * (i * D + t)], hi = (T)op.hval[2 * (i * D + t) + 1];
-      const V v = self[c + j * D];
-      cr += hr * v.x - hi * v.y;
-      ci += hr * v.y + hi * v.x;
-    }
-    const int nj = op.hnnz[j];
-    for (int t = 0; t < nj; ++t) {            // (X H)(i, j) = sum_k X(i, k) conj(H(j, k))
-      const int c = op.hcol[j * D + t];
-      const T hr = (T)op.hval[2 * (j * D + t)], hi = -(T)op.hval[2 * (j * D + t) + 1];
-      const V v = self[i + c * D];
-      cr -= v.x * hr - v.y * hi;
-      ci -= v.x * hi + v.y * hr;
-    }
-    ar[k] = gr * xe.x - gi * xe.y - hs * ci;
-    ai[k] = gr * xe.y + gi * xe.x + hs * cr;
-  }
-
-  // couplings: the entry two ahead and the record one ahead are loaded while
-  // the current neighbour is gathered
-  const int64_t p0 = op.rowptr[a], p1 = op.rowptr[a + 1];
-  DevEntry en_next{}, en_after{};
-  DevRec rc_next{};
-  if (p0 < p1) {
-    en_next = op.ent[p0];
-    rc_next = op.rec[en_next.rec];
-  }
-  if (p0 + 1 < p1) en_after = op.ent[p0 + 1];
-  for (int64_t p = p0; p < p1; ++p) {
-    const DevEntry en = en_next;
-    const DevRec rc = rc_next;
-    if (p + 1 < p1) {
-      en_next = en_after;
-      rc_next = op.rec[en_next.rec];
-      if (p + 2 < p1) en_after = op.ent[p + 2];
-    }
-    const V* __restrict__ xn = xv + (int64_t)en.nbr * E;
-    const bool dag = en.flags & 1;
-    const T cLr = (en.flags & 2) ? -(T)rc.cLr : (T)rc.cLr;
-    const T cLi = (en.flags & 2) ? -(T)rc.cLi : (T)rc.cLi;
-    const T cRr = (en.flags & 4) ? -(T)rc.cRr : (T)rc.cRr;
-    const T cRi = (en.flags & 4) ? -(T)rc.cRi : (T)rc.cRi;
-    const bool zchk = TRANS && en.nbr == trace_pos;
-    const int8_t* mL = &sop[(rc.opL < 0 ? 0 : rc.opL) * 4 * D];
-    const int8_t* mR = &sop[(rc.opR < 0 ? 0 : rc.opR) * 4 * D];
-#pragma unroll
-    for (int k = 0; k < EPT; ++k) {
-      const int e = lane + k * LANES;
-      const int i = e % D, j = e / D;
-      const int pl = rc.opL >= 0 ? mL[i] : -1;
-      if (pl >= 0) {
-        const int idx = dag ? (j + pl * D) : (pl + j * D);
-        V v = xn[idx];
-        if (dag) v.y = -v.y;
-        if (zchk && idx == op.trace_elem) { v.x = 0; v.y = 0; }
-        const T s = (T)mL[D + i];
-        ar[k] += s * (cLr * v.x - cLi * v.y);
-        ai[k] += s * (cLr * v.y + cLi * v.x);
-      }
-      const int pr = rc.opR >= 0 ? mR[2 * D + j] : -1;
-      if (pr >= 0) {
-        const int idx = dag ? (pr + i * D) : (i + pr * D);
-        V v = xn[idx];
-        if (dag) v.y = -v.y;
-        if (zchk && idx == op.trace_elem) { v.x = 0; v.y = 0; }
-        const T s = (T)mR[3 * D + j];
-        ar[k] += s * (cRr * v.x - cRi * v.y);
-        ai[k] += s * (cRr * v.y + cRi * v.x);
-      }
-    }
-  }
-  int tpar = 0;
-  if (project) {
-    int n = 0;
-    while (n + 1 < op.tb.ntier && op.tb.first[n + 1] <= a) ++n;
-    tpar = n & 1;
-  }
   V* __restrict__ yv = reinterpret_cast<V*>(y);
-#pragma unroll
-  for (int k = 0; k < EPT; ++k) {
-    const int e = lane + k * LANES;
-    V o;
-    o.x = ar[k];
-    o.y = ai[k];
-    if (project && ((op.parity[e % D] + op.parity[e / D] + tpar) & 1)) { o.x = 0; o.y = 0; }
-    yv[a * E + e] = o;
+  tab.stage(op);
+
+  if ((int64_t)blockIdx.x < n_heavy) {   // block-uniform
+    const int64_t a = blockIdx.x;
+    for (int e = tid; e < E; e += 256) {
+      V v = xv[a * E + e];
+      if (TRANS && a == trace_pos && e == op.trace_elem) v = V{0, 0};
+      xs[e] = v;
+    }
+    const T gr = (T)op.gam[2 * a], gi = (T)op.gam[2 * a + 1];
+    const int64_t p0 = op.rowptr[a], p1 = op.rowptr[a + 1];
+    const int tpar = project ? tier_parity<T>(op, a) : 0;
+    for (int k = 0; k < EPT; ++k) {
+      const int e = lane + k * LANES;
+      T ar = 0, ai = 0;
+      for (int64_t q0 = p0; q0 < p1; q0 += kStage) {
+        const int n = (int)(p1 - q0 < kStage ? p1 - q0 : kStage);
+        __syncthreads();   // the previous stage is read
+        if (tid < n) s_c[tid] = to_coupling<T>(op, op.ent[q0 + tid]);
+        __syncthreads();
+        for (int c0 = slot; c0 < n; c0 += APB * U) {
+          const int nv = (n - c0 + APB - 1) / APB;
+          add_couplings<D, T, TRANS, U>(s_c + c0, APB, nv < U ? nv : U, tab.smap, xv, e % D, e / D, trace_pos,
+                                        op.trace_elem, ar, ai);
+        }
+      }
+      __syncthreads();   // xs and the tables are staged (also for an ADO without couplings)
+      if (slot == 0) tab.template same_tier<T>(op, xs, gr, gi, e % D, e / D, ar, ai);
+      if (APB > 1) {   // sum the slices (fixed pairing)
+        __syncthreads();   // slice 0 has read xs
+        xs[tid] = V{ar, ai};
+        __syncthreads();
+        for (int half = APB / 2; half > 0; half >>= 1) {
+          if (slot < half) {
+            const V o = xs[tid + half * LANES];
+            xs[tid].x += o.x;
+            xs[tid].y += o.y;
+          }
+          __syncthreads();
+        }
+        ar = xs[tid].x;
+        ai = xs[tid].y;
+      }
+      if (slot == 0) {
+        V o{ar, ai};
+        if (project && ((op.parity[e % D] + op.parity[e / D] + tpar) & 1)) o = V{0, 0};
+        yv[a * E + e] = o;
+      }
+    }
+    return;
+  }
+
+  // Light groups: the couplings of the whole run are staged first (`per` of
+  // each ADO; more than that only in a run of one, restaged chunk by chunk).
+  // A group's own elements are loaded one group ahead and staged in
+  // alternating buffers, so a group has one barrier.
+  const int64_t g0 = ((int64_t)blockIdx.x - n_heavy) * run;
+  const int64_t groups = (op.n_ado - n_heavy + APB - 1) / APB;
+  const int nr = (int)(groups - g0 < run ? groups - g0 : run);
+  const int64_t a0 = n_heavy + g0 * APB;
+  const int per = light_max < kStage / APB ? light_max : kStage / APB;
+  auto stage_light = [&](int c0) {
+    for (int k = tid; k < nr * APB * per; k += 256) {
+      const int64_t sa = a0 + k / per;
+      int64_t p = 0, pe = 0;
+      if (sa < op.n_ado) {
+        p = op.rowptr[sa] + c0 + k % per;
+        pe = op.rowptr[sa + 1];
+      }
+      s_c[k] = to_coupling<T>(op, p < pe ? op.ent[p] : DevEntry{0, 0, 0, 0xff});
+    }
+  };
+  V own{0, 0};
+  if (EPT == 1 && a0 + slot < op.n_ado) own = xv[(a0 + slot) * E + lane];
+  stage_light(0);
+  __syncthreads();   // couplings and tables are staged
+  for (int r = 0; r < nr; ++r) {
+    const int64_t a = a0 + (int64_t)r * APB + slot;
+    const bool active = a < op.n_ado;
+    const int tpar = project ? tier_parity<T>(op, a) : 0;
+    V* xr = EPT == 1 ? &xs[(r & 1) * 256] : xs;
+    if (EPT == 1) {
+      xr[tid] = TRANS && a == trace_pos && lane == op.trace_elem ? V{0, 0} : own;
+      if (r + 1 < nr && a + APB < op.n_ado) own = xv[(a + APB) * E + lane];
+    } else {
+      __syncthreads();   // the previous group has read xs
+      for (int f = tid; f < E; f += 256)
+        xs[f] = TRANS && a == trace_pos && f == op.trace_elem ? V{0, 0} : xv[a * E + f];
+    }
+    V g{0, 0};
+    if (active) g = V{(T)op.gam[2 * a], (T)op.gam[2 * a + 1]};
+    for (int k = 0; k < EPT; ++k) {
+      const int e = lane + k * LANES;
+      T ar = 0, ai = 0;
+      for (int c0 = 0; c0 < light_max; c0 += per) {
+        if (per < light_max) {   // uniform
+          __syncthreads();
+          stage_light(c0);
+          __syncthreads();
+        }
+        if (active)
+          for (int u = 0; u < per; u += UL)
+            add_couplings<D, T, TRANS, UL>(&s_c[(r * APB + slot) * per + u], 1, per - u < UL ? per - u : UL, tab.smap,
+                                           xv, e % D, e / D, trace_pos, op.trace_elem, ar, ai);
+      }
+      if (k == 0) __syncthreads();   // xs is staged
+      if (active) {
+        tab.template same_tier<T>(op, xr + slot * E, g.x, g.y, e % D, e / D, ar, ai);
+        V o{ar, ai};
+        if (project && ((op.parity[e % D] + op.parity[e / D] + tpar) & 1)) o = V{0, 0};
+        yv[a * E + e] = o;
+      }
+    }
   }
 }
 
@@ -193,6 +340,11 @@ __global__ void k_trace_trn(const T* __restrict__ w, T* __restrict__ z, int d, i
   z[2 * (i + i * d) + 1] += w[o + 1];
 }
 
+// Light workgroups take up to kLightRunMax groups each (fewer when their
+// couplings would not fit the stage) while at least kLightBlocksMin workgroups
+// remain: 16 per CU, so a run never leaves the chip idle.
+constexpr int kLightRunMax = 8, kLightBlocksMin = 4096;
+
 template <int D, typename T>
 static hipError_t launch_d(const DevOperator& op, const T* x, T* y, int64_t trace_pos, hipStream_t s,
                            bool project) {
@@ -200,12 +352,19 @@ static hipError_t launch_d(const DevOperator& op, const T* x, T* y, int64_t trac
   constexpr int LANES = E < 256 ? E : 256;
   constexpr int APB = 256 / LANES;
   if (op.n_ado <= 0) return hipSuccess;
-  const int64_t blocks = (op.n_ado + APB - 1) / APB;
+  // heavy: every tier below the top one (the only tier of a tier-0 hierarchy)
+  const int64_t n_heavy = op.tb.ntier >= 2 ? op.tb.first[op.tb.ntier - 1] : op.n_ado;
+  const int64_t groups = (op.n_ado - n_heavy + APB - 1) / APB;
+  const int64_t fit = std::max<int64_t>(1, kStage / (APB * (int64_t)op.light_max));   // runs whose couplings fit the stage
+  const int run = (int)std::min({fit, (int64_t)kLightRunMax, std::max<int64_t>(1, groups / kLightBlocksMin)});
+  const int64_t blocks = n_heavy + (groups + run - 1) / run;
   const int pj = project ? 1 : 0;
   if (op.transposed)
-    hipLaunchKernelGGL((k_apply<D, T, true>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, pj);
+    hipLaunchKernelGGL((k_apply<D, T, true>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, pj,
+                       n_heavy, run, op.light_max);
   else
-    hipLaunchKernelGGL((k_apply<D, T, false>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, pj);
+    hipLaunchKernelGGL((k_apply<D, T, false>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, pj,
+                       n_heavy, run, op.light_max);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   if (trace_pos >= 0) {

@@ -132,6 +132,10 @@ int build_entries(const Model& m, std::vector<int64_t>& rowf, std::vector<DevEnt
   }
   rowf[m.N] = (int64_t)entf.size();
   if (6 * (int64_t)M > 65535) return fail(HEOMQ_UNSUPPORTED, "too many drawers for the record table");
+  std::vector<DevRec> recs;
+  build_records(m, recs);
+  auto op_of = [&](uint16_t rec) { return recs[rec].opL < 0 ? (uint8_t)0xff : (uint8_t)recs[rec].opL; };
+  for (DevEntry& e : entf) e.op = op_of(e.rec);
   // reverse every forward entry: K <- J becomes J <- K
   rowt.assign(m.N + 1, 0);
   for (const DevEntry& e : entf) rowt[e.nbr + 1]++;
@@ -149,7 +153,7 @@ int build_entries(const Model& m, std::vector<int64_t>& rowf, std::vector<DevEnt
       t.nbr = (int32_t)g;
       t.rec = (uint16_t)((dag ? 4 + kind : 2 + kind) * M + k);
       t.flags = dag ? (uint8_t)(1 | (nR ? 2 : 0) | (nL ? 4 : 0)) : (uint8_t)((nL ? 2 : 0) | (nR ? 4 : 0));
-      t.pad = 0;
+      t.op = op_of(t.rec);
       entt[fill[e.nbr]++] = t;
     }
   return HEOMQ_OK;
@@ -190,6 +194,7 @@ void fill_op(heomq_ctx* c, OperatorTables& t, const DevBuf& rec, bool transposed
   o.transposed = transposed;
   o.parity = c->parity.as<int8_t>();
   o.tb = c->tb;
+  o.light_max = t.light_max;
   o.trace_elem = c->d * c->d - 1;
 }
 
@@ -1203,6 +1208,10 @@ int heomq_ctx_create(const heomq_model* h, int device, heomq_ctx** out) {
   HIPCHECK(upload(c->fwd.ent, entf));
   HIPCHECK(upload(c->trn.rowptr, rowt));
   HIPCHECK(upload(c->trn.ent, entt));
+  for (int64_t g = m.L >= 1 ? m.first[m.L] : m.N; g < m.N; ++g) {
+    c->fwd.light_max = std::max<int>(c->fwd.light_max, (int)(rowf[g + 1] - rowf[g]));
+    c->trn.light_max = std::max<int>(c->trn.light_max, (int)(rowt[g + 1] - rowt[g]));
+  }
   std::vector<int8_t> map;
   build_opmap(m, map);
   HIPCHECK(upload(c->opmap, map));

@@ -60,6 +60,7 @@ inline int op_up(const heomq::Model& m, int k) {    // upper-tier operator: c fo
 
 struct OperatorTables {
   DevBuf rowptr, ent, gam;
+  int light_max = 1;                 // most couplings of a top-tier ADO
   heomq::DevOperator op;
 };
 

@@ -16,7 +16,7 @@ struct DevEntry {
   int32_t nbr;
   uint16_t rec;
   uint8_t flags;   // bit0: Xt = X^H, bit1: sL = -1, bit2: sR = -1
-  uint8_t pad;
+  uint8_t op;      // the record's operator (opL = opR in every record), 0xff: none
 };
 
 struct DevRec {
@@ -48,6 +48,7 @@ struct DevOperator {
   bool transposed = false;
   const int8_t* parity = nullptr;    // electron-number parity of each Fock state [d]
   TierBounds tb{};
+  int light_max = 1;                 // most couplings of a top-tier ADO (>= 1)
   int trace_elem = 0;                // element (i + j*d) of the trace-row ADO the trace row replaces:
                                      // d*d - 1 (TFQMR convention) or 0 (BiCG convention)
 };
