@@ -222,6 +222,10 @@ hipError_t launch_offsector_any(const DevPacked& op, const double* dense, int32_
 // the diagonal's imaginary part (:330-337), mode 2 folds the upper triangle
 // onto the lower one (lower += conj(upper)^T, upper 0, diagonal real).
 hipError_t launch_bicg_tier0_packed(const DevPacked& op, double* x, int mode, hipStream_t s);
+// out = D^-1 b with the diagonal D a scaled apply of this operator divides by
+// (DevPacked::precond): the right-hand side of a Jacobi-scaled solve.
+template <typename T>
+hipError_t launch_jacobi_scale_rhs(const DevPacked& op, const T* b, T* out, hipStream_t s);
 // Hermitianise the tier-0 block of a packed vector in place.
 template <typename T>
 hipError_t launch_herm_packed(const DevPacked& op, T* x, hipStream_t s);

@@ -934,6 +934,36 @@ __global__ void k_pack(const DevPacked op, const TD* __restrict__ dense, TP* __r
   packed[2 * t + 1] = (TP)dense[2 * src + 1];
 }
 
+// out = D^-1 b, D the diagonal the scaled applies divide by (jacobi_scale):
+// the right-hand side of a Jacobi-scaled solve.  One thread per element, one
+// read and one write of the vector; once per restart.
+template <typename T>
+__global__ void k_jacobi_scale_rhs(const DevPacked op, const T* __restrict__ b, T* __restrict__ out) {
+  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= op.total) return;
+  const int64_t a = find_ado(op, g);
+  const int dd = op.d * op.d, s = op.sec[a], t = (int)(g - op.off[a]);
+  T csr = 0, csi = 0;
+  if (op.hell_w > 0) {
+    const int64_t row = (int64_t)s * dd + t;
+    for (int k = 0; k < op.hell_w; ++k)
+      if (op.hq_ell[row * op.hell_wp + k] == t) {
+        csr += (T)op.hc_ell[2 * (row * op.hell_w + k)];
+        csi += (T)op.hc_ell[2 * (row * op.hell_w + k) + 1];
+      }
+  } else {
+    for (int u = op.hrow[s * (dd + 1) + t]; u < op.hrow[s * (dd + 1) + t + 1]; ++u)
+      if (op.hq[u] == t) {
+        csr += (T)op.hc[2 * u];
+        csi += (T)op.hc[2 * u + 1];
+      }
+  }
+  T re = b[2 * g], im = b[2 * g + 1];
+  jacobi_scale<T>(op, (T)op.gam[2 * a], (T)op.gam[2 * a + 1], csr, csi, re, im);
+  out[2 * g] = re;
+  out[2 * g + 1] = im;
+}
+
 // Block-Jacobi same-tier inverse (jacobi/calc_ax_jacobi_omp.f90:276-298 on
 // tier >= 1, :95-108 on tier 0): forward half.  Thread = packed element
 // (i, j) of ADO a; the transform sums over the H-groups of i and j only.
@@ -1642,6 +1672,14 @@ hipError_t launch_unpack(const DevPacked& op, const TP* packed, TD* dense, hipSt
   return hipGetLastError();
 }
 
+template <typename T>
+hipError_t launch_jacobi_scale_rhs(const DevPacked& op, const T* b, T* out, hipStream_t s) {
+  if (op.nprob != 1) return hipErrorInvalidValue;
+  if (op.total <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_jacobi_scale_rhs<T>), dim3((unsigned)((op.total + 255) / 256)), dim3(256), 0, s, op, b, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_jacobi_fwd(const DevPacked& op, const DevJacobi& jc, const double* r, double* t, hipStream_t s) {
   if (op.total <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_jacobi_fwd, dim3((unsigned)((op.total + 255) / 256)), dim3(256), 0, s, op, jc, r, t);
@@ -1743,6 +1781,8 @@ template hipError_t launch_pack<double, double>(const DevPacked&, const double*,
 template hipError_t launch_unpack<double, double>(const DevPacked&, const double*, double*, hipStream_t);
 template hipError_t launch_pack<double, float>(const DevPacked&, const double*, float*, hipStream_t);
 template hipError_t launch_unpack<float, double>(const DevPacked&, const float*, double*, hipStream_t);
+template hipError_t launch_jacobi_scale_rhs<double>(const DevPacked&, const double*, double*, hipStream_t);
+template hipError_t launch_jacobi_scale_rhs<float>(const DevPacked&, const float*, float*, hipStream_t);
 template hipError_t launch_herm_packed<double>(const DevPacked&, double*, hipStream_t);
 template hipError_t launch_herm_packed<float>(const DevPacked&, float*, hipStream_t);
 

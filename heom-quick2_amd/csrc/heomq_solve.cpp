@@ -235,17 +235,18 @@ int chunk_graph(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, boo
 // TFQMR on A x = b with every vector and scalar on the device.  Restarts from
 // the true residual when the quasi-residual bound is met but ||b - Ax|| is not
 // below tol*||b|| (at most 3 times; stagnation stops it).
+// one_pass: no restart (an inner solve, whose caller takes the true residual).
 // mode: 0 dense vectors and the plain operator (any trace row); 1 symmetry-
 // packed vectors and the projected operator Pi*A (trace row on the tier-0
 // block), the iterate's tier-0 block re-Hermitianised at every restart.
 template <typename T>
 int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool trans, int64_t tpos,
-              double tol, int maxiter, hipStream_t st, RunStats& rs, int mode, int prec = 0) {
+              double tol, int maxiter, hipStream_t st, RunStats& rs, int mode, int prec = 0, bool one_pass = false) {
   // the iteration runs on the left-preconditioned operator M^-1 A (prec 1:
   // Jacobi scaling, 2: block Jacobi; 0: A itself); every true residual
-  // ||b - A x|| uses the operator itself.  Jacobi scaling keeps b (the
-  // callers enable it for b = e_trace, whose one element sits on the
-  // unscaled trace row); block Jacobi iterates with M^-1 b in W.bp.
+  // ||b - A x|| uses the operator itself.  Both iterate with M^-1 b in W.bp;
+  // Jacobi scaling without W.bp keeps b (b = e_trace, whose one element sits
+  // on the unscaled trace row).
   auto Ait = [&](const T* in, T* out) -> hipError_t {
     return mode == 1 ? apply_packed_T<T>(c, trans, in, out, tpos >= 0, st, prec, W.pt)
                      : apply_T<T>(c, trans, in, out, tpos, st, false);
@@ -260,6 +261,7 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
                                  "ADO-aligned inverse)");
     HIPCHECK(precond_rhs(c, b, W.bp, W.pt, st));
   }
+  if (prec == 1 && W.bp) HIPCHECK(launch_jacobi_scale_rhs<T>(trans ? c->ptrn : c->pfwd, b, W.bp, st));
   bool fuse_ok = false;
   if constexpr (std::is_same<T, double>::value) fuse_ok = mode == 1 && prec == 2 && tfq_fusable(c, trans, tpos >= 0);
   if (fuse_ok) {   // captured chunks hold the buffer's address: a new buffer retires them
@@ -317,7 +319,7 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
       HIPCHECK(Ait(x, W.ax));
       rs.applies++;
     }
-    HIPCHECK(tfq_init_r<T>(st, n, prec == 2 ? W.bp : b, W.ax, W.w, W.y2, W.d, s, part));
+    HIPCHECK(tfq_init_r<T>(st, n, prec && W.bp ? W.bp : b, W.ax, W.w, W.y2, W.d, s, part));
     TfqmrScal& hs = *reinterpret_cast<TfqmrScal*>(static_cast<char*>(c->pinned) + 1024);
     if (prec) {   // the quasi-residual bound measures the scaled residual: scale the target with it
       HIPCHECK(hipMemcpyAsync(&hs, s, sizeof(TfqmrScal), hipMemcpyDeviceToHost, st));
@@ -376,6 +378,7 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
     HIPCHECK(flush());
     base_iters = rs.iters;
     if (hs.flag == 2 && ++stalls > 3) return fail(HEOMQ_BREAKDOWN, "TFQMR breakdown");
+    if (one_pass) break;
   }
   double rr = 0, bb = 0;
   if (int rc = true_resid(rr, bb)) return rc;
@@ -512,17 +515,17 @@ int steady_solve(heomq_ctx* c, double* x, const double* b, double tol, int maxit
   }
   RunStats rs;
   // automatic choice: Jacobi scaling when H is diagonal in the occupation
-  // basis, block Jacobi otherwise
+  // basis, block Jacobi otherwise (forward solves only).  The scaling divides
+  // by the iterated operator's own diagonal, so it serves the transposed
+  // solves too: a single-impurity adjoint solve (M = 72, L = 3) takes 40
+  // iterations scaled against 330 unscaled.
   int prec = 0;
-  if (packed && !transpose) {
+  if (packed) {
     const int want = c->precond >= 0 ? c->precond : (c->h_diagonal ? 1 : 2);
-    if (want == 1 && !b) prec = 1;   // the scaling keeps only b = e_trace
-    if (want == 2) prec = 2;
+    if (want == 1 || !transpose) prec = want;
   }
-  if (prec == 2) {
-    W.pt = v[kWorkVecs + 2];
-    W.bp = v[kWorkVecs + 3];
-  }
+  if (prec == 2) W.pt = v[kWorkVecs + 2];
+  if (prec == 2 || (prec == 1 && b)) W.bp = v[kWorkVecs + 3];
   // The steady problem (b = e_trace): a few sweeps of the reference's own
   // convergent block-Jacobi iteration (trace kept) before TFQMR.  They damp
   // the start's tier-1+ residual (3e3 x ||b|| on the two-impurity model), so
@@ -612,12 +615,10 @@ int heomq_solve_steady_mixed(heomq_ctx* c, double* x, const double* b, double to
   const int64_t n = 2 * c->ptotal;
   // Preconditioning as the FP64 solver chooses it (automatic: Jacobi scaling
   // for diagonal H, block Jacobi otherwise).  The FP32 inner solves take the
-  // block-Jacobi inverse (ADO-aligned form, FP32 vectors, FP64 transform); the
-  // Jacobi scaling keeps only b = e_trace, so residual corrections of a
-  // diagonal-H model iterate unscaled.
+  // block-Jacobi inverse in its ADO-aligned form (FP32 vectors, FP64 transform).
   const int want = c->precond >= 0 ? c->precond : (c->h_diagonal ? 1 : 2);
-  const int prec32 = (want == 2 && c->pjac.ado_blocks > 0) ? 2 : 0;
-  const int prec64 = want == 2 ? 2 : 0;
+  const int prec32 = want == 2 && c->pjac.ado_blocks <= 0 ? 0 : want;
+  const int prec64 = want;
   std::vector<double*> v64;
   if (int rc = carve<double>(c->ws64, n, 3, v64)) return rc;
   std::vector<float*> v32;
@@ -626,10 +627,8 @@ int heomq_solve_steady_mixed(heomq_ctx* c, double* x, const double* b, double to
   Work<float> W{v32[0], v32[1], v32[2], v32[3], v32[4], v32[5], v32[6], v32[7]};
   float* x32 = v32[kWorkVecs];
   float* r32 = v32[kWorkVecs + 1];
-  if (prec32 == 2) {
-    W.pt = v32[kWorkVecs + 2];
-    W.bp = v32[kWorkVecs + 3];
-  }
+  if (prec32 == 2) W.pt = v32[kWorkVecs + 2];
+  if (prec32) W.bp = v32[kWorkVecs + 3];
   double* ax = v64[0];
   double* bb = v64[1];
   double* xs = v64[2];
@@ -671,7 +670,11 @@ int heomq_solve_steady_mixed(heomq_ctx* c, double* x, const double* b, double to
     HIPCHECK(vec_fill<float>(st, n, x32, 0.0f));
     RunStats rs;
     const int cap = std::min(inner_cap, maxiter - inner_total);
-    const int irc = tfqmr_run<float>(c, x32, r32, W, n, false, 0, inner_tol, cap, st, rs, 1, prec32);
+    // Jacobi-scaled: one pass of the recurrences.  FP32 restarts iterate to the
+    // cap without passing eps32 * ||A|| ||dx||; the FP64 residual above restarts
+    // instead (single impurity, M = 72, L = 3: 9.1 -> 6.2 ms; block Jacobi on
+    // two impurities with M = 64 gains nothing, 68 against 74 ms)
+    const int irc = tfqmr_run<float>(c, x32, r32, W, n, false, 0, inner_tol, cap, st, rs, 1, prec32, prec32 == 1);
     if (irc != HEOMQ_OK && irc != HEOMQ_NOT_CONVERGED) return irc;
     inner_total += rs.iters;
     applies += rs.applies;
@@ -682,10 +685,8 @@ int heomq_solve_steady_mixed(heomq_ctx* c, double* x, const double* b, double to
     std::vector<double*> w64;
     if (int e = carve<double>(c->ws64b, n, kWorkVecs + 2, w64)) return e;
     Work<double> W64{w64[0], w64[1], w64[2], w64[3], w64[4], w64[5], w64[6], w64[7]};
-    if (prec64 == 2) {
-      W64.pt = w64[kWorkVecs];
-      W64.bp = w64[kWorkVecs + 1];
-    }
+    if (prec64 == 2) W64.pt = w64[kWorkVecs];
+    if (prec64 == 2 || (prec64 == 1 && b)) W64.bp = w64[kWorkVecs + 1];
     RunStats rs;
     rc = tfqmr_run<double>(c, xs, bb, W64, n, false, 0, tol, std::max(maxiter - inner_total, 1), st, rs, 1, prec64);
     fp64_iters = rs.iters;
