@@ -330,7 +330,8 @@ struct PackedHost {
   std::vector<int32_t> block, lblock, lnz;
   int64_t n_heavy = 0, light_begin = 0;
   std::vector<DevEntryP> pentf, pentt;
-  std::vector<int32_t> maps;
+  std::vector<int2> maps;
+  bool wide = false;
   int tslot = -1;
   int max_light[2] = {0, 0};
   // grouped heavy rows (per operator) and sector-batched top-tier blocks
@@ -515,10 +516,10 @@ int finish_packed_host(const Model& m, const std::vector<int64_t>& rowf, const s
   if (lnz.empty()) lnz.push_back(0);
   // paired gather maps: output slot t of sector s -> the signed slots in the
   // neighbour (sector s2) of its left-operator and right-operator terms
-  std::vector<int32_t> maps;
+  std::vector<int2> maps((size_t)dd, make_int2(kMapAbsent, kMapAbsent));   // the map without terms
   std::map<std::tuple<int, int, int, int, int>, int32_t> mapidx;
   auto side_value = [&](int s, int s2, int o, int dag, int side, int t) -> int {
-    if (o < 0) return 0;
+    if (o < 0) return kMapAbsent;
     const int8_t* pL = &omap[(size_t)o * 4 * d];
     const int8_t* sL = pL + d;
     const int8_t* pR = pL + 2 * d;
@@ -527,14 +528,14 @@ int finish_packed_host(const Model& m, const std::vector<int64_t>& rowf, const s
     const int i = e % d, j = e / d;
     if (side == 0) {
       const int pl = pL[i];
-      if (pl < 0) return 0;
+      if (pl < 0) return kMapAbsent;
       const int q = pos[(size_t)s2 * dd + (dag ? (j + pl * d) : (pl + j * d))];
-      return q >= 0 ? (q + 1) * sL[i] : 0;
+      return q >= 0 ? 16 * q + (sL[i] < 0 ? 1 : 0) : kMapAbsent;
     }
     const int pr = pR[j];
-    if (pr < 0) return 0;
+    if (pr < 0) return kMapAbsent;
     const int q = pos[(size_t)s2 * dd + (dag ? (pr + i * d) : (i + pr * d))];
-    return q >= 0 ? (q + 1) * sR[j] : 0;
+    return q >= 0 ? 16 * q + (sR[j] < 0 ? 1 : 0) : kMapAbsent;
   };
   auto getmap = [&](int s, int s2, int oL, int oR, int dag) -> int32_t {
     const auto key = std::make_tuple(s, s2, oL, oR, dag);
@@ -544,8 +545,8 @@ int finish_packed_host(const Model& m, const std::vector<int64_t>& rowf, const s
     bool any = false;
     for (int t = 0; t < nnz[s]; ++t) {
       const int vl = side_value(s, s2, oL, dag, 0, t), vr = side_value(s, s2, oR, dag, 1, t);
-      any |= (vl != 0 || vr != 0);
-      maps.push_back((int32_t)((uint32_t)(uint16_t)(int16_t)vl | ((uint32_t)(uint16_t)(int16_t)vr << 16)));
+      any |= (vl != kMapAbsent || vr != kMapAbsent);
+      maps.push_back(make_int2(vl, vr));
     }
     const int32_t res = any ? at : -1;
     if (!any) maps.resize(at);
@@ -572,7 +573,6 @@ int finish_packed_host(const Model& m, const std::vector<int64_t>& rowf, const s
   if (too_many) return fail(HEOMQ_UNSUPPORTED, "packed layout: gather maps exceed 2^31 entries");
   group_heavy_rows(rowf, ph.pentf, nnz, n_heavy, ph.hg_off[0], ph.hg[0]);
   if (both) group_heavy_rows(rowt, ph.pentt, nnz, n_heavy, ph.hg_off[1], ph.hg[1]);
-  if (maps.empty()) maps.push_back(0);
   ph.off = std::move(off);
   ph.total = total;
   ph.block = std::move(block);
@@ -581,6 +581,9 @@ int finish_packed_host(const Model& m, const std::vector<int64_t>& rowf, const s
   ph.n_heavy = n_heavy;
   ph.light_begin = light_begin;
   ph.maps = std::move(maps);
+  // HEOMQ_WIDE=1 takes the 64-bit gathers on any layout (for comparison)
+  const char* wide = std::getenv("HEOMQ_WIDE");
+  ph.wide = total > kNarrowElems || (int64_t)ph.maps.size() > ((int64_t)1 << 28) || (wide && wide[0] == '1');
   ph.tslot = ph.pos[(size_t)ph.sec[0] * dd + (d - 1) + (d - 1) * d];
   for (int w = 0; w < (both ? 2 : 1); ++w) {
     const auto& rows = w == 0 ? rowf : rowt;
@@ -683,7 +686,8 @@ int build_packed(heomq_ctx* c, const Model& m, const std::vector<int64_t>& rowf,
     p.rowptr = (w == 0 ? c->fwd.rowptr : c->trn.rowptr).as<int64_t>();
     p.ent = (w == 0 ? c->p_entf : c->p_entt).as<DevEntryP>();
     p.trace_slot = ph.tslot;
-    p.maps = c->p_maps.as<int32_t>();
+    p.maps = c->p_maps.as<int2>();
+    p.wide = ph.wide ? 1 : 0;
     p.n_heavy = ph.n_heavy;
     p.light_begin = ph.light_begin;
     p.light_block_ado = c->p_lblock.as<int32_t>();
@@ -691,12 +695,14 @@ int build_packed(heomq_ctx* c, const Model& m, const std::vector<int64_t>& rowf,
     p.max_light_couplings = ph.max_light[w];
     p.n_lt_blocks = (int)ph.lt_blk.size();
     p.lt_u = ph.lt_u;
-    // the default form: the sector-batched top tier with the sliced heavy
-    // rows (the fastest on both test workloads' forward applies); the
-    // autotuner (heomq_ctx_autotune) picks per operator, HEOMQ_APPLY_FORM
-    // forces one
+    // the default form: the sector-batched top tier; below it one wave per ADO
+    // where every sector is small (the single impurity: 36.8 against 89.2 us in
+    // form 2 at M = 72, L = 4, 6.8 against 8.4 at L = 3), else the grouped rows
+    // (two impurities, M = 112, L = 3: 50.5 against 56.2 us, 14.5 against 16.5
+    // at M = 64).  The autotuner (heomq_ctx_autotune) picks per operator,
+    // HEOMQ_APPLY_FORM forces one.
     const char* form = std::getenv("HEOMQ_APPLY_FORM");
-    set_apply_form(c, w, form ? std::atoi(form) : 2);
+    set_apply_form(c, w, form ? std::atoi(form) : (c->heavy_wave_ok ? 6 : 3));
   }
   return HEOMQ_OK;
 }
@@ -854,7 +860,8 @@ int build_spa_operator(heomq_ctx* c, const int32_t* nnz_spa, const std::vector<i
   p.rowptr = c->fwd.rowptr.as<int64_t>();
   p.ent = so.ent.as<DevEntryP>();
   p.trace_slot = -1;
-  p.maps = so.maps.as<int32_t>();
+  p.maps = so.maps.as<int2>();
+  p.wide = ph.wide ? 1 : 0;
   p.n_heavy = ph.n_heavy;
   p.light_begin = ph.light_begin;
   p.light_block_ado = so.lblock.as<int32_t>();
@@ -989,7 +996,8 @@ int build_trun(heomq_ctx* c) {
   p.ent = tr.ent.as<DevEntryP>();
   p.gam = tr.gam.as<double>();
   p.trace_slot = ph.tslot;
-  p.maps = tr.maps.as<int32_t>();
+  p.maps = tr.maps.as<int2>();
+  p.wide = ph.wide ? 1 : 0;
   p.n_heavy = ph.n_heavy;
   p.light_begin = ph.light_begin;
   p.light_block_ado = tr.lblock.as<int32_t>();

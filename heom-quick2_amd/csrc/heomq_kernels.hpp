@@ -64,12 +64,19 @@ struct DevOperator {
 struct DevEntryP {       // packed coupling (16 bytes)
   int32_t base;          // neighbour's first packed element
   int32_t map;           // offset of the paired gather map (output slot -> two signed neighbour
-                         // slots, left and right operator, as int16 halves); -1: no term
+                         // slots, left and right operator); -1: no term
   int32_t ncls;          // the neighbour's sector (host-side table building only)
   uint16_t rec;          // coefficient record (cL, cR)
   uint8_t flags;         // bit0 X^H, bit1 sL = -1, bit2 sR = -1
   uint8_t pad;
 };
+
+// One side of a gather-map pair: 16 times the neighbour slot | sign in bit 0,
+// or kMapAbsent.  The first d * d pairs of a table are the map without terms.
+constexpr int32_t kMapAbsent = 0x40000000;
+// Vectors of up to this many elements are gathered at 32-bit byte offsets
+// below kMapAbsent (16 bytes an element)
+constexpr int64_t kNarrowElems = (int64_t)1 << 26;
 
 // LDS limits of the restructured packed apply (checked when its tables are built)
 constexpr int kHeavyStage = 256;   // entries of one heavy row staged at once
@@ -130,7 +137,7 @@ struct DevPacked {
   int n_lt_blocks = 0;
   int lt_u = 0;
   // slot-space tables: i(HX - XH) per sector as CSR over packed slots, and the
-  // gather maps (value (q + 1) * sign, 0 = no term) referenced by entries
+  // gather maps (kMapAbsent: no term) referenced by entries
   // the same rows padded to a fixed width hell_w (slot -1 / coefficient 0 as
   // padding) when every row is short: index loads then depend only on (s, t)
   int hell_w = 0;                    // 0: use the CSR form
@@ -140,7 +147,8 @@ struct DevPacked {
   const int32_t* hrow = nullptr;     // [S][d*d + 1] row starts into hq / hc
   const int16_t* hq = nullptr;
   const double* hc = nullptr;        // complex coefficients of i(HX - XH)
-  const int32_t* maps = nullptr;     // paired gather maps (int16 left | int16 right << 16)
+  const int2* maps = nullptr;        // paired gather maps {left, right}
+  int wide = 0;                      // 1: more than kNarrowElems elements, gathered at 64-bit addresses
   // batch of problems sharing every structural table (grid y = problem):
   // problem p's vectors start p * vstride complex elements in, its records,
   // ADO rates and commutator coefficients p * rec_stride / gam_stride /

@@ -11,6 +11,7 @@
 // element.  The output is the projected operator Pi*A: off-sector elements do
 // not exist and the tier-0 block is Hermitianised by a one-block fix-up.
 #include <algorithm>
+#include <type_traits>
 
 #include "heomq_kernels.hpp"
 #include "heomq_shadow.hpp"
@@ -47,6 +48,57 @@ __device__ inline typename P2<T>::type ldw(const typename P2<T>::type* __restric
   if (s_x != nullptr && r >= 0 && r < win_n) return s_x[r];
   return ld<T, TRANS>(xv, g, zero_at);
 }
+
+// The elements couplings gather from x.  A map value is one side of a
+// coupling's gather: 16 times the neighbour slot, bit 0 the sign, kMapAbsent
+// when there is no term (no load is issued: about half of the lanes' terms
+// are absent at d = 16, and the address path is one of the kernel's bounds).
+// Up to kNarrowElems elements (not WIDE) the address is a 32-bit byte offset
+// from x, one instruction; larger vectors take 64-bit addresses.
+template <typename T, bool WIDE>
+struct XSrc {
+  using V = typename P2<T>::type;
+  const V* __restrict__ p;
+  __device__ explicit XSrc(const V* x) : p(x) {}
+  __device__ V operator()(int32_t base, int32_t m) const {
+    if (m >= kMapAbsent) return V{0, 0};
+    if (WIDE) return p[(int64_t)base + (m >> 4)];
+    uint32_t off = ((uint32_t)base << 4) + (uint32_t)(m & ~15);
+    if (sizeof(V) == 8) off >>= 1;
+    return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + off);
+  }
+};
+
+// v with its sign bit flipped by the top bit of s
+__device__ inline double flip(double v, uint32_t s) { return __hiloint2double(__double2hiint(v) ^ (int)s, __double2loint(v)); }
+__device__ inline float flip(float v, uint32_t s) { return __int_as_float(__float_as_int(v) ^ (int)s); }
+
+// A coupling's gather with the map pair m, conjugated (cj = 1 << 31) for X^H:
+// the signed elements of the left and right operator.
+template <typename T, bool TRANS, bool WIDE>
+__device__ inline typename P2<T>::type gather(const XSrc<T, WIDE>& x, int32_t base, int32_t m, int64_t zero_at) {
+  typename P2<T>::type v = x(base, m);
+  if (TRANS && m < kMapAbsent && base + (m >> 4) == (int32_t)zero_at) { v.x = 0; v.y = 0; }
+  return v;
+}
+// a += c * (the gathered element with its map sign and conjugation)
+template <typename T>
+__device__ inline void mac_signed(typename P2<T>::type c, typename P2<T>::type v, int32_t m, uint32_t cj, T& ar, T& ai) {
+  const uint32_t sg = (uint32_t)m << 31;
+  const T x = flip(v.x, sg), y = flip(v.y, sg ^ cj);
+  ar += c.x * x;
+  ar -= c.y * y;
+  ai += c.x * y;
+  ai += c.y * x;
+}
+template <bool WIDE>
+__device__ inline int2 map_at(const int2* __restrict__ maps, int map, int t) {
+  if (WIDE) return maps[(int64_t)map + t];
+  return *reinterpret_cast<const int2*>(reinterpret_cast<const char*>(maps) + (uint32_t)((map + t) << 3));
+}
+// t / w for t <= 256, 1 <= w <= 256 (exact: t (inv w - 65536) < 65536)
+__device__ inline int div_inv(int w) { return (int)(65536.0f * __frcp_rn((float)w)) + 1; }
+__device__ inline int div_by(int t, int inv) { return (int)(((uint32_t)t * (uint32_t)inv) >> 16); }
 
 // A Chebyshev term applied where the apply writes its output (no y in
 // memory): with y = L p1 for element g,  p[g] += a y;  x[g] += b p[g]
@@ -85,7 +137,7 @@ template <typename T, bool TRANS>
 __device__ inline void diag_term(const DevPacked& op, const double* __restrict__ hc_ell,
                                  const typename P2<T>::type* __restrict__ xv, T gr, T gi,
                                  int64_t base, int s, int t, int64_t zero_at, T& ar, T& ai,
-                                 const typename P2<T>::type* s_x, int64_t win_lo, int win_n, T& csr, T& csi) {
+                                 const typename P2<T>::type* s_x, int64_t win_lo, int win_n, bool scaled, T& csr, T& csi) {
   using V = typename P2<T>::type;
   const int dd = op.d * op.d;
   const V xe = ldw<T, TRANS>(xv, base + t, zero_at, s_x, win_lo, win_n);
@@ -110,7 +162,7 @@ __device__ inline void diag_term(const DevPacked& op, const double* __restrict__
         const V v = ldw<T, TRANS>(xv, base + q, zero_at, s_x, win_lo, win_n);
         cr += (T)h.x * v.x - (T)h.y * v.y;
         ci += (T)h.x * v.y + (T)h.y * v.x;
-        if (q == t) { csr += (T)h.x; csi += (T)h.y; }
+        if (scaled && q == t) { csr += (T)h.x; csi += (T)h.y; }
       }
     }
   } else {
@@ -120,7 +172,7 @@ __device__ inline void diag_term(const DevPacked& op, const double* __restrict__
       const T hr = (T)op.hc[2 * u], hi = (T)op.hc[2 * u + 1];
       cr += hr * v.x - hi * v.y;
       ci += hr * v.y + hi * v.x;
-      if (op.hq[u] == t) { csr += hr; csi += hi; }
+      if (scaled && op.hq[u] == t) { csr += hr; csi += hi; }
     }
   }
   const T hs = (T)op.hsign;
@@ -149,95 +201,135 @@ __device__ inline CoefLR load_coef(const DevRec* rec, int k) {
   return CoefLR{p[0], p[1]};
 }
 
-// U couplings at once: every entry's paired gather-map value (one 32-bit load
-// for the left and right operator), then every neighbour element, are loaded
-// before any of them is used.
-template <typename T, bool TRANS, int U>
-__device__ inline void coupling_block(const DevEntryP* en, const CoefLR* cf, int nvalid,
-                                      const int32_t* __restrict__ maps, const typename P2<T>::type* __restrict__ xv,
-                                      int t, int64_t zero_at, T& ar, T& ai) {
+// U couplings at once: every entry's gather-map pair, then every neighbour
+// element, are loaded before any of them is used.
+template <typename T, bool TRANS, bool WIDE, int U>
+__device__ inline void coupling_block(const DevEntryP* en, const CoefLR* cf, int nvalid, const int2* __restrict__ maps,
+                                      const XSrc<T, WIDE>& xs, int t, int64_t zero_at, T& ar, T& ai) {
   using V = typename P2<T>::type;
-  int mL[U], mR[U];
+  int2 mv[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int mv = (u < nvalid && en[u].map >= 0) ? maps[en[u].map + t] : 0;
-    mL[u] = (int)(int16_t)(mv & 0xffff);
-    mR[u] = (int)(int16_t)((uint32_t)mv >> 16);
-  }
+  for (int u = 0; u < U; ++u)
+    mv[u] = (u < nvalid && en[u].map >= 0) ? map_at<WIDE>(maps, en[u].map, t) : make_int2(kMapAbsent, kMapAbsent);
   V vL[U], vR[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int64_t b = u < nvalid ? (int64_t)en[u].base : 0;
-    vL[u] = mL[u] != 0 ? ld<T, TRANS>(xv, b + (mL[u] > 0 ? mL[u] : -mL[u]) - 1, zero_at) : V{0, 0};
-    vR[u] = mR[u] != 0 ? ld<T, TRANS>(xv, b + (mR[u] > 0 ? mR[u] : -mR[u]) - 1, zero_at) : V{0, 0};
+    const int32_t b = u < nvalid ? en[u].base : 0;
+    vL[u] = gather<T, TRANS, WIDE>(xs, b, mv[u].x, zero_at);
+    vR[u] = gather<T, TRANS, WIDE>(xs, b, mv[u].y, zero_at);
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    if (mL[u] == 0 && mR[u] == 0) continue;
-    const uint8_t fl = en[u].flags;
-    const T cj = (fl & 1) ? (T)-1 : (T)1;   // X^H: conjugate the gathered element
-    const T sL = ((mL[u] > 0) != ((fl & 2) != 0)) ? (T)1 : (T)-1;
-    const T sR = ((mR[u] > 0) != ((fl & 4) != 0)) ? (T)1 : (T)-1;
-    const T lx = vL[u].x, ly = cj * vL[u].y, rx = vR[u].x, ry = cj * vR[u].y;
-    const T clr = (T)cf[u].l.x, cli = (T)cf[u].l.y, crr = (T)cf[u].r.x, cri = (T)cf[u].r.y;
-    ar += sL * (clr * lx - cli * ly) + sR * (crr * rx - cri * ry);
-    ai += sL * (clr * ly + cli * lx) + sR * (crr * ry + cri * rx);
+    if (u >= nvalid) break;
+    const uint32_t fl = en[u].flags, cj = fl << 31;
+    V cl, cr;
+    cl.x = flip((T)cf[u].l.x, (fl << 30) & 0x80000000u);
+    cl.y = flip((T)cf[u].l.y, (fl << 30) & 0x80000000u);
+    cr.x = flip((T)cf[u].r.x, (fl << 29) & 0x80000000u);
+    cr.y = flip((T)cf[u].r.y, (fl << 29) & 0x80000000u);
+    mac_signed<T>(cl, vL[u], mv[u].x, cj, ar, ai);
+    mac_signed<T>(cr, vR[u], mv[u].y, cj, ar, ai);
   }
 }
 
-// One coupling's contribution from its gathered elements (signs in the map
-// values and the entry flags, coefficients cL, cR).
+// A coupling staged in LDS: the coefficients with the entry's signs, its
+// neighbour's first element, and its map | dagger << 31 (map 0 is the map
+// without terms).
 template <typename T>
-__device__ inline void coupling_accum(int mL, int mR, typename P2<T>::type vL, typename P2<T>::type vR, uint8_t fl,
-                                      const CoefLR& cf, T& ar, T& ai) {
-  if (mL == 0 && mR == 0) return;
-  const T cj = (fl & 1) ? (T)-1 : (T)1;
-  const T sL = ((mL > 0) != ((fl & 2) != 0)) ? (T)1 : (T)-1;
-  const T sR = ((mR > 0) != ((fl & 4) != 0)) ? (T)1 : (T)-1;
-  const T lx = vL.x, ly = cj * vL.y, rx = vR.x, ry = cj * vR.y;
-  const T clr = (T)cf.l.x, cli = (T)cf.l.y, crr = (T)cf.r.x, cri = (T)cf.r.y;
-  ar += sL * (clr * lx - cli * ly) + sR * (crr * rx - cri * ry);
-  ai += sL * (clr * ly + cli * lx) + sR * (crr * ry + cri * rx);
-}
+struct StagedLds {
+  typename P2<T>::type* l;
+  typename P2<T>::type* r;
+  int2* bm;
+  __device__ void put(int k, const DevEntryP& e, const DevRec* rec) const {
+    const CoefLR c = e.map >= 0 ? load_coef(rec, e.rec) : CoefLR{};
+    const T sl = (e.flags & 2) ? (T)-1 : (T)1, sr = (e.flags & 4) ? (T)-1 : (T)1;
+    typename P2<T>::type v;
+    v.x = sl * (T)c.l.x;
+    v.y = sl * (T)c.l.y;
+    l[k] = v;
+    v.x = sr * (T)c.r.x;
+    v.y = sr * (T)c.r.y;
+    r[k] = v;
+    bm[k] = make_int2(e.base, (e.map >= 0 ? e.map : 0) | ((e.flags & 1) ? (int)0x80000000 : 0));
+  }
+};
 
-// The couplings k0, k0 + S, k0 + 2S, ... of a heavy lane with the entries and
-// coefficients staged in LDS, U per batch, software-pipelined: the gather-map
-// values of batch b + 1 are loaded while batch b's elements are in flight, so
-// each batch waits for one global load instead of two (map, then element).
-template <typename T, bool TRANS, int U>
-__device__ inline void staged_couplings(const DevEntryP* s_en, const CoefLR* s_cf, int nent, int k0, int S,
-                                        const int32_t* __restrict__ maps, const typename P2<T>::type* __restrict__ xv,
-                                        int t, int64_t zero_at, T& ar, T& ai) {
+// The staged couplings k0, k0 + S, k0 + 2S, ... below nent of one lane, U per
+// batch, software-pipelined: the map values of batch b + 1 are loaded while
+// batch b's elements are in flight, so each batch waits for one global load
+// instead of two (map, then element).
+template <typename T, bool TRANS, bool WIDE, int U>
+__device__ inline void staged_couplings(const StagedLds<T>& st, int nent, int k0, int S, const int2* __restrict__ maps,
+                                        const XSrc<T, WIDE>& xs, int t, int64_t zero_at, T& ar, T& ai) {
   using V = typename P2<T>::type;
-  int mv[U];
+  int2 bm[U], mv[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int k = k0 + u * S;
-    mv[u] = (k < nent && s_en[k].map >= 0) ? maps[s_en[k].map + t] : 0;
+    bm[u] = st.bm[k < nent ? k : k0];
+    mv[u] = k < nent ? map_at<WIDE>(maps, bm[u].y & 0x7fffffff, t) : make_int2(kMapAbsent, kMapAbsent);
   }
   for (; k0 < nent; k0 += S * U) {
     V vL[U], vR[U];
-    int mL[U], mR[U];
+    int2 mc[U];
+    uint32_t cj[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * S;
-      const int64_t b = k < nent ? (int64_t)s_en[k].base : 0;
-      mL[u] = (int)(int16_t)(mv[u] & 0xffff);
-      mR[u] = (int)(int16_t)((uint32_t)mv[u] >> 16);
-      vL[u] = mL[u] != 0 ? ld<T, TRANS>(xv, b + (mL[u] > 0 ? mL[u] : -mL[u]) - 1, zero_at) : V{0, 0};
-      vR[u] = mR[u] != 0 ? ld<T, TRANS>(xv, b + (mR[u] > 0 ? mR[u] : -mR[u]) - 1, zero_at) : V{0, 0};
+      vL[u] = gather<T, TRANS, WIDE>(xs, bm[u].x, mv[u].x, zero_at);
+      vR[u] = gather<T, TRANS, WIDE>(xs, bm[u].x, mv[u].y, zero_at);
+      mc[u] = mv[u];
+      cj[u] = (uint32_t)bm[u].y & 0x80000000u;
     }
     const int kn = k0 + S * U;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = kn + u * S;
-      mv[u] = (k < nent && s_en[k].map >= 0) ? maps[s_en[k].map + t] : 0;
+      if (k < nent) {
+        bm[u] = st.bm[k];
+        mv[u] = map_at<WIDE>(maps, bm[u].y & 0x7fffffff, t);
+      } else {
+        mv[u] = make_int2(kMapAbsent, kMapAbsent);
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = k0 + u * S;
-      if (k < nent) coupling_accum<T>(mL[u], mR[u], vL[u], vR[u], s_en[k].flags, s_cf[k], ar, ai);
+      __builtin_amdgcn_sched_barrier(0);   // one coupling's coefficients in registers at a time
+      if (k < nent) {
+        mac_signed<T>(st.l[k], vL[u], mc[u].x, cj[u], ar, ai);
+        mac_signed<T>(st.r[k], vR[u], mc[u].y, cj[u], ar, ai);
+      }
     }
+  }
+}
+
+// U staged couplings from k of one lane (nv of them valid), nothing prefetched.
+template <typename T, bool TRANS, bool WIDE, int U>
+__device__ inline void staged_block(const StagedLds<T>& st, int k, int nv, const int2* __restrict__ maps,
+                                    const XSrc<T, WIDE>& xs, int t, int64_t zero_at, T& ar, T& ai) {
+  using V = typename P2<T>::type;
+  int2 mv[U];
+  int32_t base[U];
+  uint32_t cj[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int2 bm = st.bm[u < nv ? k + u : k];
+    base[u] = bm.x;
+    cj[u] = (uint32_t)bm.y & 0x80000000u;
+    mv[u] = u < nv ? map_at<WIDE>(maps, bm.y & 0x7fffffff, t) : make_int2(kMapAbsent, kMapAbsent);
+  }
+  V vL[U], vR[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    vL[u] = gather<T, TRANS, WIDE>(xs, base[u], mv[u].x, zero_at);
+    vR[u] = gather<T, TRANS, WIDE>(xs, base[u], mv[u].y, zero_at);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u >= nv) break;
+    __builtin_amdgcn_sched_barrier(0);   // one coupling's coefficients in registers at a time
+    mac_signed<T>(st.l[k + u], vL[u], mv[u].x, cj[u], ar, ai);
+    mac_signed<T>(st.r[k + u], vR[u], mv[u].y, cj[u], ar, ai);
   }
 }
 
@@ -253,11 +345,12 @@ constexpr size_t kAlign16(size_t b) { return (b + 15) / 16 * 16; }
 constexpr size_t kLightOffP0 = kAlign16(257 * 8), kLightOffP1 = kLightOffP0 + kAlign16(257 * 8),
                  kLightOffSec = kLightOffP1 + kAlign16(257 * 8), kLightOffGam = kLightOffSec + kAlign16(257 * 4),
                  kLightOffX = kLightOffGam + kAlign16(257 * 16), kLightSmem = kLightOffX + 256 * 16;
-constexpr size_t kHeavyOffRi = 256 * 8, kHeavyOffEn = 2 * 256 * 8, kHeavyOffCf = kHeavyOffEn + 256 * sizeof(DevEntryP),
-                 kHeavyOffX = kHeavyOffCf + 256 * sizeof(CoefLR), kHeavySmem = kHeavyOffX + 256 * 16;
+constexpr size_t kHeavyOffRi = 256 * 8, kHeavyOffL = 2 * 256 * 8, kHeavyOffR = kHeavyOffL + 256 * 16,
+                 kHeavyOffBm = kHeavyOffR + 256 * 16, kHeavyOffX = kHeavyOffBm + 256 * 8,
+                 kHeavySmem = kHeavyOffX + 256 * 16;
 constexpr size_t kApplySmem0 = kLightSmem > kHeavySmem ? kLightSmem : kHeavySmem;
 
-template <typename T, bool TRANS, int U, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool EPI = false>
 __device__ inline void light_body(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x, T* __restrict__ y,
                                   int64_t zero_at, int bid, char* smem, bool scaled, const ChebEpi* ep = nullptr) {
   using V = typename P2<T>::type;
@@ -268,6 +361,8 @@ __device__ inline void light_body(const DevPacked& op, const Coefs cf_p, const T
   double2* s_gam = reinterpret_cast<double2*>(smem + kLightOffGam);
   V* s_x = reinterpret_cast<V*>(smem + kLightOffX);
   const V* __restrict__ xv = reinterpret_cast<const V*>(x);
+  const XSrc<T, WIDE> xs(xv);
+  constexpr int U = 2;
   const int lo = op.light_block_ado[bid], hi = op.light_block_ado[bid + 1];
   const int cnt = hi - lo + 1;
   for (int k = threadIdx.x; k < cnt; k += 256) {
@@ -294,7 +389,7 @@ __device__ inline void light_body(const DevPacked& op, const Coefs cf_p, const T
   const int64_t p0 = s_p0[l], p1 = s_p1[l];
   T ar, ai, csr, csi;
   diag_term<T, TRANS>(op, cf_p.hc_ell, xv, (T)s_gam[l].x, (T)s_gam[l].y, base, s_sec[l], slot, zero_at, ar, ai,
-                      s_x, win_lo, win_n, csr, csi);
+                      s_x, win_lo, win_n, scaled, csr, csi);
   for (int64_t p = p0; p < p1; p += U) {
     const int nv = (int)(p1 - p < U ? p1 - p : U);
     DevEntryP en[U];
@@ -309,7 +404,7 @@ __device__ inline void light_body(const DevPacked& op, const Coefs cf_p, const T
         cf[u] = CoefLR{};
       }
     }
-    coupling_block<T, TRANS, U>(en, cf, nv, op.maps, xv, slot, zero_at, ar, ai);
+    coupling_block<T, TRANS, WIDE, U>(en, cf, nv, op.maps, xs, slot, zero_at, ar, ai);
   }
   if (scaled) jacobi_scale<T>(op, (T)s_gam[l].x, (T)s_gam[l].y, csr, csi, ar, ai);
   if (EPI) {
@@ -342,7 +437,7 @@ struct StageOut {
 // coupling of the ADO (entries and coefficients staged in LDS), two
 // couplings per step; the slices are summed through LDS in a fixed order.
 // Block 0 (the tier-0 ADO) then applies the trace row and Hermitianises.
-template <typename T, bool TRANS, bool STAGE = false, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool STAGE = false, bool EPI = false>
 __device__ inline void heavy_body(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x, T* __restrict__ y,
                                   int64_t zero_at, int rdo, int bid, char* smem, bool scaled,
                                   StageOut* so = nullptr, const ChebEpi* ep = nullptr) {
@@ -350,8 +445,8 @@ __device__ inline void heavy_body(const DevPacked& op, const Coefs cf_p, const T
   constexpr int kStage = 256;
   T* red_r = reinterpret_cast<T*>(smem);
   T* red_i = reinterpret_cast<T*>(smem + kHeavyOffRi);
-  DevEntryP* s_en = reinterpret_cast<DevEntryP*>(smem + kHeavyOffEn);
-  CoefLR* s_cf = reinterpret_cast<CoefLR*>(smem + kHeavyOffCf);
+  const StagedLds<T> st{reinterpret_cast<V*>(smem + kHeavyOffL), reinterpret_cast<V*>(smem + kHeavyOffR),
+                        reinterpret_cast<int2*>(smem + kHeavyOffBm)};
   V* s_x = reinterpret_cast<V*>(smem + kHeavyOffX);
   const int64_t a = bid;
   const int64_t base = op.off[a];
@@ -362,27 +457,23 @@ __device__ inline void heavy_body(const DevPacked& op, const Coefs cf_p, const T
   const int64_t p0 = op.rowptr[a], p1 = op.rowptr[a + 1];
   const int nent = (int)(p1 - p0);
   const bool staged = nent <= kStage;
-  if (staged)
-    for (int k = threadIdx.x; k < nent; k += 256) {
-      const DevEntryP e0 = op.ent[p0 + k];
-      s_en[k] = e0;
-      s_cf[k] = load_coef(cf_p.rec, e0.rec);
-    }
+  if (staged && threadIdx.x < nent) st.put(threadIdx.x, op.ent[p0 + threadIdx.x], cf_p.rec);
+  const XSrc<T, WIDE> xs(xv);
   const int win_n = nnz < 256 ? nnz : 256;
   if (threadIdx.x < win_n) s_x[threadIdx.x] = ld<T, TRANS>(xv, base + threadIdx.x, zero_at);
   __syncthreads();
   constexpr int U = 2;
   for (int t0 = 0; t0 < nnz; t0 += 256) {   // nnz is uniform over the block: every thread takes the same trips
     const int w = nnz - t0 < 256 ? nnz - t0 : 256;   // slots in this pass
-    const int S = 256 / w;
-    const int lane = threadIdx.x % w, slice = threadIdx.x / w;
+    const int inv = div_inv(w), S = div_by(256, inv);
+    const int slice = div_by(threadIdx.x, inv), lane = threadIdx.x - slice * w;
     const int t = t0 + lane;
     T ar = 0, ai = 0, csr = 0, csi = 0;
     if (slice < S) {
       if (slice == 0)
-        diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, ar, ai, s_x, base, win_n, csr, csi);
+        diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, ar, ai, s_x, base, win_n, scaled, csr, csi);
       if (staged) {
-        staged_couplings<T, TRANS, U>(s_en, s_cf, nent, slice, S, op.maps, xv, t, zero_at, ar, ai);
+        staged_couplings<T, TRANS, WIDE, U>(st, nent, slice, S, op.maps, xs, t, zero_at, ar, ai);
       } else {   // entries from global memory (ADOs with more than 256 couplings)
         for (int k0 = slice; k0 < nent; k0 += S * U) {
           DevEntryP en[U];
@@ -400,7 +491,7 @@ __device__ inline void heavy_body(const DevPacked& op, const Coefs cf_p, const T
               cf[u] = CoefLR{};
             }
           }
-          coupling_block<T, TRANS, U>(en, cf, nv, op.maps, xv, t, zero_at, ar, ai);
+          coupling_block<T, TRANS, WIDE, U>(en, cf, nv, op.maps, xs, t, zero_at, ar, ai);
         }
       }
     }
@@ -470,10 +561,10 @@ constexpr size_t kGOffB = 256 * sizeof(HWgt<double>);                           
 constexpr size_t kGOffG = kGOffB + 2 * 16 * (size_t)kHeavyPairs;                   // run table
 constexpr size_t kGSmem = kGOffG + 16 * (size_t)(kHeavyGroups + 1);
 
-template <typename T, bool TRANS, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool STAGE = false, bool EPI = false>
 __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x,
                                      T* __restrict__ y, int64_t zero_at, int rdo, int bid, char* smem, bool scaled,
-                                     const ChebEpi* ep = nullptr) {
+                                     StageOut* so = nullptr, const ChebEpi* ep = nullptr) {
   using V = typename P2<T>::type;
   HWgt<T>* s_w = reinterpret_cast<HWgt<T>*>(smem);
   V* s_B = reinterpret_cast<V*>(smem + kGOffB);
@@ -506,38 +597,46 @@ __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, cons
     s_w[k] = w;
   }
   __syncthreads();
-  // phase 1: the runs' accumulators in neighbour slot space
+  // phase 1: the runs' accumulators in neighbour slot space; with P <= 128
+  // pairs each run is cut into NS = 256 / P parts (at most 4), a lane per
+  // (part, pair), so that every lane works and a run's chain is shorter
   const int P = s_g[ng].w;
-  for (int l = threadIdx.x; l < P; l += 256) {
+  const int NS = P > 128 ? 1 : (P > 64 ? 2 : 4);
+  const XSrc<T, WIDE> xs(xv);
+  for (int l = threadIdx.x; l < P * NS; l += 256) {
+    const int part = (l >= P) + (l >= 2 * P) + (l >= 3 * P), pr = NS == 1 ? l : l - part * P;
     int lo = 0, hi = ng - 1;
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
-      if ((s_g[mid].w & 0x7fffffff) <= l) lo = mid; else hi = mid - 1;
+      if ((s_g[mid].w & 0x7fffffff) <= pr) lo = mid; else hi = mid - 1;
     }
     const int4 G = s_g[lo];
-    const int u = l - (G.w & 0x7fffffff);
+    const int u = pr - (G.w & 0x7fffffff), u16 = u << 4;
+    const int len = G.y - G.x, g0e = G.x - (int)p0;
+    int e = NS == 1 ? g0e : g0e + ((len * part) >> (NS >> 1));
+    const int e1 = NS == 1 ? g0e + len : g0e + ((len * (part + 1)) >> (NS >> 1));
     T lr = 0, li = 0, rr = 0, ri = 0;
-    int e = G.x;
-    for (; e + 4 <= G.y; e += 4) {   // four independent loads in flight
+    for (; e < e1; e += 4) {   // up to four independent loads in flight
       V v[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = ld<T, TRANS>(xv, (int64_t)s_w[e + q - p0].base + u, zero_at);
+      for (int q = 0; q < 4; ++q) {
+        v[q] = V{0, 0};
+        if (e + q < e1) v[q] = gather<T, TRANS, WIDE>(xs, s_w[e + q].base, u16, zero_at);
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const HWgt<T>& w = s_w[e + q - p0];
-        lr += w.lr * v[q].x - w.li * v[q].y;
-        li += w.lr * v[q].y + w.li * v[q].x;
-        rr += w.rr * v[q].x - w.ri * v[q].y;
-        ri += w.rr * v[q].y + w.ri * v[q].x;
+        if (e + q >= e1) break;
+        __builtin_amdgcn_sched_barrier(0);   // one weight in registers at a time
+        const HWgt<T>& w = s_w[e + q];
+        lr += w.lr * v[q].x;
+        lr -= w.li * v[q].y;
+        li += w.lr * v[q].y;
+        li += w.li * v[q].x;
+        rr += w.rr * v[q].x;
+        rr -= w.ri * v[q].y;
+        ri += w.rr * v[q].y;
+        ri += w.ri * v[q].x;
       }
-    }
-    for (; e < G.y; ++e) {
-      const V v = ld<T, TRANS>(xv, (int64_t)s_w[e - p0].base + u, zero_at);
-      const HWgt<T>& w = s_w[e - p0];
-      lr += w.lr * v.x - w.li * v.y;
-      li += w.lr * v.y + w.li * v.x;
-      rr += w.rr * v.x - w.ri * v.y;
-      ri += w.rr * v.y + w.ri * v.x;
     }
     V bl, br;
     bl.x = lr; bl.y = li;
@@ -550,31 +649,30 @@ __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, cons
   // in the sliced form (fixed pairing)
   for (int t0 = 0; t0 < nnz; t0 += 256) {
     const int w = nnz - t0 < 256 ? nnz - t0 : 256;
-    const int S = 256 / w;
-    const int lane = threadIdx.x % w, slice = threadIdx.x / w;
+    const int inv = div_inv(w), S = div_by(256, inv);
+    const int slice = div_by(threadIdx.x, inv), lane = threadIdx.x - slice * w;
     const int t = t0 + lane;
     T ar = 0, ai = 0, csr = 0, csi = 0;
     if (slice < S) {
       if (slice == 0)
-        diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, ar, ai, nullptr, 0, 0, csr, csi);
+        diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, ar, ai, nullptr, 0, 0, scaled, csr, csi);
       for (int g = slice; g < ng; g += S) {
         const int4 G = s_g[g];
         const int ub = G.w & 0x7fffffff;
-        const T cj = G.w < 0 ? (T)-1 : (T)1;   // X^H run: conj of the accumulator
-        const int mv = op.maps[G.z + t];
-        const int mL = (int)(int16_t)(mv & 0xffff), mR = (int)(int16_t)((uint32_t)mv >> 16);
-        if (mL != 0) {
-          const V b = s_B[2 * (ub + (mL > 0 ? mL : -mL) - 1)];
-          const T sg = mL > 0 ? (T)1 : (T)-1;
-          ar += sg * b.x;
-          ai += sg * cj * b.y;
-        }
-        if (mR != 0) {
-          const V b = s_B[2 * (ub + (mR > 0 ? mR : -mR) - 1) + 1];
-          const T sg = mR > 0 ? (T)1 : (T)-1;
-          ar += sg * b.x;
-          ai += sg * cj * b.y;
-        }
+        const uint32_t cj = (uint32_t)G.w & 0x80000000u;   // X^H run: conj of the accumulator
+        const int2 mv = map_at<WIDE>(op.maps, G.z, t);
+        if (mv.x < kMapAbsent)
+          for (int q = 0; q < NS; ++q) {   // the run's parts
+            const V b = s_B[2 * (q * P + ub + (mv.x >> 4))];
+            ar += flip(b.x, (uint32_t)mv.x << 31);
+            ai += flip(b.y, ((uint32_t)mv.x << 31) ^ cj);
+          }
+        if (mv.y < kMapAbsent)
+          for (int q = 0; q < NS; ++q) {
+            const V b = s_B[2 * (q * P + ub + (mv.y >> 4)) + 1];
+            ar += flip(b.x, (uint32_t)mv.y << 31);
+            ai += flip(b.y, ((uint32_t)mv.y << 31) ^ cj);
+          }
       }
     }
     red_r[threadIdx.x] = ar;
@@ -595,14 +693,27 @@ __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, cons
       V o;
       o.x = sr;
       o.y = si;
-      if (EPI)
+      if (STAGE) {   // one pass (nnz <= 256): slot t = threadIdx.x
+        so->v = make_double2((double)sr, (double)si);
+        so->act = true;
+      } else if (EPI) {
         cheb_put(ep, base + t, (double)sr, (double)si);
-      else
+      } else {
         reinterpret_cast<V*>(y)[base + t] = o;
+      }
     }
     __syncthreads();
   }
-  if (a == 0) tier0_fixup_block<T>(op, x, y, rdo);   // block-uniform branch
+  if (STAGE) {
+    so->gbase = base;
+    so->lbase = 0;
+    so->t = threadIdx.x;
+    so->s = s;
+    so->gr = (double)gr;
+    so->gi = (double)gi;
+  } else if (a == 0 && !EPI) {   // (with the epilogue no trace row and no Hermitian fix-up: host check)
+    tier0_fixup_block<T>(op, x, y, rdo);   // block-uniform branch
+  }
 }
 
 // Heavy ADOs of small sectors (at most 16 elements, e.g. every ADO of the
@@ -611,7 +722,7 @@ __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, cons
 // of two w, so 64 / w slices walk the coupling list (entries, records and
 // gather maps from global memory, two couplings in flight); the slices are
 // summed by shuffles in a fixed tree, with no LDS and no barrier.
-template <typename T, bool TRANS, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool EPI = false>
 __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x, T* __restrict__ y,
                                   int64_t zero_at, int64_t a, bool scaled, const ChebEpi* ep = nullptr) {
   using V = typename P2<T>::type;
@@ -619,11 +730,11 @@ __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T
   const int64_t base = op.off[a];
   const int nnz = (int)(op.off[a + 1] - base);
   if (nnz == 0) return;   // wave-uniform
-  int w = 1;
-  while (w < nnz) w <<= 1;   // <= kHeavyWaveMaxNnz (host check)
-  const int S = 64 / w, slice = lane / w, t = lane - slice * w;
+  const int sh = 32 - __clz(nnz - 1 > 0 ? nnz - 1 : 0), w = 1 << sh;   // slots rounded up: <= kHeavyWaveMaxNnz (host check)
+  const int S = 64 >> sh, slice = lane >> sh, t = lane & (w - 1);
   const bool act = t < nnz;
   const V* __restrict__ xv = reinterpret_cast<const V*>(x);
+  const XSrc<T, WIDE> xs(xv);
   const int s = op.sec[a];
   const T gr = (T)cf_p.gam[2 * a], gi = (T)cf_p.gam[2 * a + 1];
   const int64_t p0 = op.rowptr[a];
@@ -631,7 +742,7 @@ __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T
   T ar = 0, ai = 0, csr = 0, csi = 0;
   if (act) {
     if (slice == 0)
-      diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, ar, ai, nullptr, 0, 0, csr, csi);
+      diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, ar, ai, nullptr, 0, 0, scaled, csr, csi);
     constexpr int U = 2;
     for (int k0 = slice; k0 < nent; k0 += S * U) {
       DevEntryP en[U];
@@ -649,7 +760,7 @@ __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T
           cf[u] = CoefLR{};
         }
       }
-      coupling_block<T, TRANS, U>(en, cf, nv, op.maps, xv, t, zero_at, ar, ai);
+      coupling_block<T, TRANS, WIDE, U>(en, cf, nv, op.maps, xs, t, zero_at, ar, ai);
     }
   }
   // lane = slice * w + t: shuffles by multiples of w fold the slices onto slice 0
@@ -671,44 +782,65 @@ __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T
 }
 
 // Top tier, sector-batched: a block takes 256 / nnz top-tier ADOs of one
-// sector, one lane per (ADO, slot).  Each lane loads its ADO's first element,
-// rate and couplings from the block's own tables (one level below the block
-// descriptor), then every coupling's map value and record, then the lower-tier
-// elements, and sums the couplings before any barrier; only its own element
-// of x goes through LDS, where the sector's commutator rows (staged once per
-// block) read their neighbours.  Four levels of dependent loads in all.
-constexpr size_t kLOffHc = 256 * 2, kLOffX = kLOffHc + 256 * 16, kLSmem = kLOffX + 256 * 16;
+// sector, one lane per (ADO, slot).  A lane needs its ADO's first element,
+// rate and couplings, every coupling's map value and coefficients, and the
+// lower-tier elements.  With several lanes per ADO (kLStage couplings or fewer
+// per block) the couplings and rates are loaded once per ADO into LDS, with
+// the entries' signs on the coefficients, and the lanes read them there: 12
+// global loads per lane instead of 25 at d = 16, where the loads' address
+// path, not their bytes, was the bound.  With few lanes per ADO (d = 4) each
+// lane loads its own.  The lane's own element of x goes through LDS, where the
+// sector's commutator rows (staged once per block) read their neighbours.
+constexpr int kLStage = 128;   // couplings of one block staged in LDS
+constexpr int kLightU = 3;     // of one lane in flight
+constexpr size_t kLOffHc = 0, kLOffX = kLOffHc + 256 * 16, kLOffL = kLOffX + 256 * 16,
+                 kLOffR = kLOffL + kLStage * 16, kLOffBm = kLOffR + kLStage * 16, kLOffG = kLOffBm + kLStage * 8,
+                 kLSmem = kLOffG + kLStage * 16;
 
-template <typename T, bool TRANS, bool STAGE = false, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool STAGE = false, bool EPI = false>
 __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x,
                                     T* __restrict__ y, int64_t zero_at, int bid, char* smem, bool scaled,
                                     StageOut* so = nullptr, const ChebEpi* ep = nullptr) {
   using V = typename P2<T>::type;
-  int16_t* s_hq = reinterpret_cast<int16_t*>(smem);
   double2* s_hc = reinterpret_cast<double2*>(smem + kLOffHc);
   V* s_x = reinterpret_cast<V*>(smem + kLOffX);
+  const StagedLds<T> st{reinterpret_cast<V*>(smem + kLOffL), reinterpret_cast<V*>(smem + kLOffR),
+                        reinterpret_cast<int2*>(smem + kLOffBm)};
+  V* s_g = reinterpret_cast<V*>(smem + kLOffG);
   const V* __restrict__ xv = reinterpret_cast<const V*>(x);
+  const XSrc<T, WIDE> xs(xv);
   const int4 bd = op.lt_blk[bid];
   const int cnt = bd.y, nnz = bd.z, s = bd.w, U = op.lt_u;
   const int dd = op.d * op.d;
   const int W = op.hell_w;
+  const bool stg = cnt * U <= kLStage;        // block-uniform
   const bool hst = W > 0 && nnz * W <= 256;   // the sector's commutator rows fit the LDS table
-  if (hst)
-    for (int k = threadIdx.x; k < nnz * W; k += 256) {
-      const int row = k / W, kk = k - row * W;
-      const int64_t r0 = (int64_t)s * dd + row;
-      s_hq[k] = op.hq_ell[r0 * op.hell_wp + kk];
-      s_hc[k] = reinterpret_cast<const double2*>(cf_p.hc_ell)[r0 * W + kk];
-    }
-  const int j = threadIdx.x / nnz, t = threadIdx.x - j * nnz;   // nnz >= 1 (host check)
+  const int j = div_by(threadIdx.x, div_inv(nnz)), t = threadIdx.x - j * nnz;   // 1 <= nnz <= 256 (host check)
   const bool act = j < cnt;
   const int64_t i = (int64_t)bd.x + j;
-  int64_t base = 0;
+  int32_t base = 0;
   T ar = 0, ai = 0, gr = 0, gi = 0;
-  if (act) {
-    base = op.lt_off[i];
+  DevEntryP e0{0, -1, -1, 0, 0, 0};
+  int ida = 0;
+  if (stg) {
+    if (threadIdx.x < cnt * U) e0 = op.lt_ent[(int64_t)bd.x * U + threadIdx.x];
+    if (threadIdx.x < cnt) ida = op.lt_id[bd.x + threadIdx.x];
+  }
+  if (act) base = op.lt_off[i];
+  if (hst && threadIdx.x < nnz * W)   // rows of one sector are consecutive
+    s_hc[threadIdx.x] = reinterpret_cast<const double2*>(cf_p.hc_ell)[(int64_t)s * dd * W + threadIdx.x];
+  if (act) s_x[threadIdx.x] = ld<T, TRANS>(xv, (int64_t)base + t, zero_at);
+  if (stg) {
+    if (threadIdx.x < cnt * U) st.put(threadIdx.x, e0, cf_p.rec);
+    if (threadIdx.x < cnt) {
+      const double2 g = reinterpret_cast<const double2*>(cf_p.gam)[ida];
+      V gv;
+      gv.x = (T)g.x;
+      gv.y = (T)g.y;
+      s_g[threadIdx.x] = gv;
+    }
+  } else if (act) {
     const int64_t a = op.lt_id[i];
-    s_x[threadIdx.x] = ld<T, TRANS>(xv, base + t, zero_at);
     gr = (T)cf_p.gam[2 * a];
     gi = (T)cf_p.gam[2 * a + 1];
     // the lower-tier couplings, two at a time: entries, then map values and
@@ -716,31 +848,22 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
     const DevEntryP* en = op.lt_ent + i * U;
     for (int r0 = 0; r0 < U; r0 += 2) {
       DevEntryP e[2];
-      int mv[2];
       CoefLR cf[2];
 #pragma unroll
       for (int q = 0; q < 2; ++q) e[q] = r0 + q < U ? en[r0 + q] : DevEntryP{0, -1, -1, 0, 0, 0};
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        mv[q] = e[q].map >= 0 ? op.maps[e[q].map + t] : 0;
-        cf[q] = e[q].map >= 0 ? load_coef(cf_p.rec, e[q].rec) : CoefLR{};
-      }
-      V vl[2], vr[2];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int mL = (int)(int16_t)(mv[q] & 0xffff), mR = (int)(int16_t)((uint32_t)mv[q] >> 16);
-        vl[q] = mL != 0 ? ld<T, TRANS>(xv, (int64_t)e[q].base + (mL > 0 ? mL : -mL) - 1, zero_at) : V{0, 0};
-        vr[q] = mR != 0 ? ld<T, TRANS>(xv, (int64_t)e[q].base + (mR > 0 ? mR : -mR) - 1, zero_at) : V{0, 0};
-      }
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int mL = (int)(int16_t)(mv[q] & 0xffff), mR = (int)(int16_t)((uint32_t)mv[q] >> 16);
-        coupling_accum<T>(mL, mR, vl[q], vr[q], e[q].flags, cf[q], ar, ai);
-      }
+      for (int q = 0; q < 2; ++q) cf[q] = e[q].map >= 0 ? load_coef(cf_p.rec, e[q].rec) : CoefLR{};
+      coupling_block<T, TRANS, WIDE, 2>(e, cf, 2, op.maps, xs, t, zero_at, ar, ai);
     }
   }
   __syncthreads();
   if (!act) return;   // after the only barrier
+  if (stg) {
+    gr = s_g[j].x;
+    gi = s_g[j].y;
+    for (int r0 = 0; r0 < U; r0 += kLightU)
+      staged_block<T, TRANS, WIDE, kLightU>(st, j * U + r0, U - r0, op.maps, xs, t, zero_at, ar, ai);
+  }
   T csr = 0, csi = 0;
   const V* xw = s_x + j * nnz;   // this ADO's elements
   if (hst) {
@@ -748,20 +871,30 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
     ar += gr * xe.x - gi * xe.y;
     ai += gr * xe.y + gi * xe.x;
     T cr = 0, ci = 0;
-    for (int k = 0; k < W; ++k) {
-      const int q = s_hq[t * W + k];
-      const double2 h = s_hc[t * W + k];
-      const V v = xw[q];
-      cr += (T)h.x * v.x - (T)h.y * v.y;
-      ci += (T)h.x * v.y + (T)h.y * v.x;
-      if (q == t) { csr += (T)h.x; csi += (T)h.y; }
+    const int4* qrow = reinterpret_cast<const int4*>(op.hq_ell + ((int64_t)s * dd + t) * op.hell_wp);
+    const double2* hrow = s_hc + t * W;
+    for (int k0 = 0; k0 < W; k0 += 8) {
+      const int4 qq = qrow[k0 >> 3];
+      const int packed[4] = {qq.x, qq.y, qq.z, qq.w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (k0 + k >= W) break;
+        const int q = (packed[k >> 1] >> ((k & 1) * 16)) & 0xffff;   // slots are >= 0
+        const double2 h = hrow[k0 + k];
+        const V v = xw[q];
+        cr += (T)h.x * v.x;
+        cr -= (T)h.y * v.y;
+        ci += (T)h.x * v.y;
+        ci += (T)h.y * v.x;
+        if (scaled && q == t) { csr += (T)h.x; csi += (T)h.y; }
+      }
     }
     const T hs = (T)op.hsign;
     ar += hs * cr;
     ai += hs * ci;
   } else {
     T dr, di;
-    diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, dr, di, xw, base, nnz, csr, csi);
+    diag_term<T, TRANS>(op, cf_p.hc_ell, xv, gr, gi, base, s, t, zero_at, dr, di, xw, base, nnz, scaled, csr, csi);
     ar += dr;
     ai += di;
   }
@@ -778,13 +911,13 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
     return;
   }
   if (EPI) {
-    cheb_put(ep, base + t, (double)ar, (double)ai);
+    cheb_put(ep, (int64_t)base + t, (double)ar, (double)ai);
     return;
   }
   V o;
   o.x = ar;
   o.y = ai;
-  reinterpret_cast<V*>(y)[base + t] = o;
+  reinterpret_cast<V*>(y)[(int64_t)base + t] = o;
 }
 
 // One launch for the whole apply: blocks [0, n_heavy) take the ADOs below the
@@ -796,7 +929,13 @@ constexpr size_t kApplySmem1 = kGSmem > kLSmem ? kGSmem : kLSmem;
 constexpr size_t kApplySmem = kApplySmem0 > kApplySmem1 ? kApplySmem0 : kApplySmem1;
 
 // Block bx of problem p of the apply (the kernels below supply the two).
-template <typename T, bool TRANS, int U, bool EPI = false>
+// FORM >= 0: the operator's form (apply_form) at compile time, so that a kernel
+// holds only its own bodies' registers; kAnyForm: read from the operator.
+constexpr int kAnyForm = -1;
+static int apply_form(const DevPacked& op) {
+  return (op.hg_off ? 1 : 0) | (op.lt_blk ? 2 : 0) | (op.heavy_wave ? 4 : 0);
+}
+template <typename T, bool TRANS, bool WIDE, int FORM, bool EPI = false>
 __device__ inline void apply_block(const DevPacked& op, int64_t p, int64_t bx, const T* __restrict__ x,
                                    T* __restrict__ y, int64_t zero_at, int rdo, char* smem,
                                    const ChebEpi* ep = nullptr) {
@@ -805,45 +944,48 @@ __device__ inline void apply_block(const DevPacked& op, int64_t p, int64_t bx, c
   x += 2 * p * op.vstride;
   y += 2 * p * op.vstride;
   const Coefs cf{op.rec + p * op.rec_stride, op.gam + 2 * p * op.gam_stride, op.hc_ell + 2 * p * op.hc_stride};
+  const bool wave = FORM < 0 ? op.heavy_wave != 0 : (FORM & 4) != 0;
+  const bool grouped = FORM < 0 ? op.hg_off != nullptr : (FORM & 1) != 0;
+  const bool sector = FORM < 0 ? op.lt_blk != nullptr : (FORM & 2) != 0;
   const int64_t hb = heavy_blocks(op);
   if (bx < hb) {   // block-uniform
-    if (op.heavy_wave && bx > 0) {   // four ADOs of small sectors, a wave each (no barrier)
+    if (wave && bx > 0) {   // four ADOs of small sectors, a wave each (no barrier)
       const int64_t a = 1 + (bx - 1) * 4 + (threadIdx.x >> 6);
-      if (a < op.n_heavy) heavy_wave<T, TRANS, EPI>(op, cf, x, y, zero_at, a, scaled, ep);
+      if (a < op.n_heavy) heavy_wave<T, TRANS, WIDE, EPI>(op, cf, x, y, zero_at, a, scaled, ep);
       return;
     }
     const int a = (int)bx;
-    if (op.hg_off && op.hg_off[a + 1] > op.hg_off[a])
-      heavy_grouped<T, TRANS, EPI>(op, cf, x, y, zero_at, rdo, a, smem, scaled, ep);
+    if (grouped && op.hg_off[a + 1] > op.hg_off[a])
+      heavy_grouped<T, TRANS, WIDE, false, EPI>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
     else
-      heavy_body<T, TRANS, false, EPI>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
-  } else if (op.lt_blk) {
-    light_sector<T, TRANS, false, EPI>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, nullptr, ep);
+      heavy_body<T, TRANS, WIDE, false, EPI>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
+  } else if (sector) {
+    light_sector<T, TRANS, WIDE, false, EPI>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, nullptr, ep);
   } else {
-    light_body<T, TRANS, U, EPI>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, ep);
+    light_body<T, TRANS, WIDE, EPI>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, ep);
   }
 }
 
-template <typename T, bool TRANS, int U>
+template <typename T, bool TRANS, bool WIDE, int FORM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 k_apply_packed(const DevPacked op, const T* __restrict__ x, T* __restrict__ y, int64_t zero_at, int rdo) {
   __shared__ __align__(16) char smem[kApplySmem];
-  apply_block<T, TRANS, U>(op, blockIdx.y, blockIdx.x, x, y, zero_at, rdo, smem);   // grid y: problem of a batch
+  apply_block<T, TRANS, WIDE, FORM>(op, blockIdx.y, blockIdx.x, x, y, zero_at, rdo, smem);   // grid y: problem of a batch
 }
 
 // One Chebyshev term in one launch: the forward apply of p1 (no trace row,
 // no Hermitian fix-up) with each output element folded into the recurrence
 // and the sum at once (ChebEpi); L p1 itself is never stored.
-template <int U>
+template <bool WIDE, int FORM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 k_apply_packed_cheb(const DevPacked op, const double* __restrict__ p1, const ChebEpi ep) {
   __shared__ __align__(16) char smem[kApplySmem];
-  apply_block<double, false, U, true>(op, 0, blockIdx.x, p1, nullptr, -1, 0, smem, &ep);
+  apply_block<double, false, WIDE, FORM, true>(op, 0, blockIdx.x, p1, nullptr, -1, 0, smem, &ep);
 }
 
 // Forward applies of problems of several shapes in one flat grid (the shapes
 // come largest first, so their long heavy workgroups are dispatched first).
-template <typename T, int U>
+template <typename T, bool WIDE, int FORM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 k_apply_packed_multi(const ApplyMulti am, const T* __restrict__ x, T* __restrict__ y, int rdo) {
   __shared__ __align__(16) char smem[kApplySmem];
@@ -853,7 +995,7 @@ k_apply_packed_multi(const ApplyMulti am, const T* __restrict__ x, T* __restrict
   const int64_t loc = b - am.bstart[g], j = loc / am.nb[g];
   const int64_t p = am.pmap[g] ? am.pmap[g][j] : j;
   const DevPacked& op = am.ops[g];
-  apply_block<T, false, U>(op, p, loc - j * am.nb[g], x + op.xoff, y + op.xoff, -1, rdo, smem);
+  apply_block<T, false, WIDE, FORM>(op, p, loc - j * am.nb[g], x + op.xoff, y + op.xoff, -1, rdo, smem);
 }
 
 // Tier-0 fix-ups (one block): trace row (forward: y(d,d) = tr x0; transposed:
@@ -1322,7 +1464,7 @@ __global__ __launch_bounds__(256) void k_jacobi_ado(const DevPacked op, const De
 // ep.prev_out[k ceil(gridDim.x / 16) + blockIdx.x]; EP 2, out =
 // aw = M^-1 A w and the partial rt.aw at ep.partial[blockIdx.x].  Nothing
 // runs once the problem's flag is set.
-template <bool RU, int EP>
+template <bool RU, int EP, bool WIDE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 k_apply_packed_jac(const DevPacked op, const DevJacobi jc, const double* __restrict__ x, double* __restrict__ out,
                    int rdo, const TfqEpi ep) {
@@ -1338,10 +1480,12 @@ k_apply_packed_jac(const DevPacked op, const DevJacobi jc, const double* __restr
   so.v = make_double2(0.0, 0.0);
   so.lbase = 0;
   so.t = 0;
-  if (heavy)
-    heavy_body<double, false, true>(op, cf, x, nullptr, -1, rdo, (int)blockIdx.x, smem, false, &so);
+  if (heavy && op.hg_off && op.hg_off[blockIdx.x + 1] > op.hg_off[blockIdx.x])
+    heavy_grouped<double, false, WIDE, true>(op, cf, x, nullptr, -1, rdo, (int)blockIdx.x, smem, false, &so);
+  else if (heavy)
+    heavy_body<double, false, WIDE, true>(op, cf, x, nullptr, -1, rdo, (int)blockIdx.x, smem, false, &so);
   else
-    light_sector<double, false, true>(op, cf, x, nullptr, -1, (int)(blockIdx.x - hb), smem, false, &so);
+    light_sector<double, false, WIDE, true>(op, cf, x, nullptr, -1, (int)(blockIdx.x - hb), smem, false, &so);
   __syncthreads();   // the apply's LDS is free from here
   double2* xw = reinterpret_cast<double2*>(smem);
   double2* tw = xw + 256;
@@ -1582,18 +1726,20 @@ static hipError_t launch_p(const DevPacked& op, const T* x, T* y, bool rdo, hipS
   const int64_t blocks = apply_blocks(op);
   if (blocks > 0) {
     const dim3 grid((unsigned)blocks, (unsigned)op.nprob);
-    const int u = op.max_light_couplings;
     const int r = rdo ? 1 : 0;
-#define HEOMQ_APPLY(UU)                                                                                  \
-  do {                                                                                                   \
-    if (op.transposed)                                                                                   \
-      hipLaunchKernelGGL((k_apply_packed<T, true, UU>), grid, dim3(256), 0, s, op, x, y, zero_at, r);    \
-    else                                                                                                 \
-      hipLaunchKernelGGL((k_apply_packed<T, false, UU>), grid, dim3(256), 0, s, op, x, y, zero_at, r);   \
-  } while (0)
-    if (u <= 1) HEOMQ_APPLY(1);
-    else HEOMQ_APPLY(2);
-#undef HEOMQ_APPLY
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, op, x, y, zero_at, r); };
+    auto pick = [&](auto trans) {
+      constexpr bool TR = decltype(trans)::value;
+      if (op.wide) return go(k_apply_packed<T, TR, true, kAnyForm>);
+      switch (apply_form(op)) {
+        case 2: return go(k_apply_packed<T, TR, false, 2>);
+        case 3: return go(k_apply_packed<T, TR, false, 3>);
+        case 6: return go(k_apply_packed<T, TR, false, 6>);
+        default: return go(k_apply_packed<T, TR, false, kAnyForm>);
+      }
+    };
+    if (op.transposed) pick(std::true_type{});
+    else pick(std::false_type{});
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
@@ -1622,17 +1768,34 @@ hipError_t launch_apply_packed_cheb(const DevPacked& op, const double* p1, doubl
   const int64_t blocks = apply_blocks(op);
   if (blocks <= 0) return hipSuccess;
   const ChebEpi ep{p, x, a, b};
-  if (op.max_light_couplings <= 1)
-    hipLaunchKernelGGL((k_apply_packed_cheb<1>), dim3((unsigned)blocks), dim3(256), 0, s, op, p1, ep);
-  else
-    hipLaunchKernelGGL((k_apply_packed_cheb<2>), dim3((unsigned)blocks), dim3(256), 0, s, op, p1, ep);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, op, p1, ep); };
+  if (op.wide) {
+    go(k_apply_packed_cheb<true, kAnyForm>);
+  } else {
+    switch (apply_form(op)) {
+      case 2: go(k_apply_packed_cheb<false, 2>); break;
+      case 3: go(k_apply_packed_cheb<false, 3>); break;
+      case 6: go(k_apply_packed_cheb<false, 6>); break;
+      default: go(k_apply_packed_cheb<false, kAnyForm>);
+    }
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_apply_packed_multi_f64(const ApplyMulti& am, const double* x, double* y, bool rdo, hipStream_t s) {
   if (am.ng < 1 || am.ng > kApplyShapesPerLaunch || am.bstart[am.ng] <= 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_apply_packed_multi<double, 2>), dim3((unsigned)am.bstart[am.ng]), dim3(256), 0, s, am, x, y,
-                     rdo ? 1 : 0);
+  bool wide = false;
+  int form = apply_form(am.ops[0]);
+  for (int g = 0; g < am.ng; ++g) {
+    wide = wide || am.ops[g].wide;
+    if (apply_form(am.ops[g]) != form) form = kAnyForm;
+  }
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)am.bstart[am.ng]), dim3(256), 0, s, am, x, y, rdo ? 1 : 0);
+  };
+  if (wide) go(k_apply_packed_multi<double, true, kAnyForm>);
+  else if (form == 6) go(k_apply_packed_multi<double, false, 6>);
+  else go(k_apply_packed_multi<double, false, kAnyForm>);
   return hipGetLastError();
 }
 hipError_t launch_apply_packed_f32(const DevPacked& op, const float* x, float* y, bool rdo, hipStream_t s) {
@@ -1728,22 +1891,27 @@ hipError_t launch_jacobi_ado_f32(const DevPacked& op, const DevJacobi& jc, const
 }
 
 bool apply_jac_fusable(const DevPacked& op, const DevJacobi& jc) {
-  return op.lt_blk != nullptr && !op.heavy_wave && op.hg_off == nullptr && !op.transposed && op.precond == 0 &&
+  return op.lt_blk != nullptr && !op.heavy_wave && !op.transposed && op.precond == 0 &&
          op.nprob == 1 && op.n_heavy > 0 && op.d <= 16 && jc.ado_blocks > 0 && jc.desc != nullptr;
+}
+
+template <int EP>
+static hipError_t launch_jac(const DevPacked& op, const DevJacobi& jc, const double* x, double* y, bool rdo,
+                             const TfqEpi& ep, int64_t blocks, hipStream_t s) {
+  const int r = rdo ? 1 : 0;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, op, jc, x, y, r, ep);
+    return hipGetLastError();
+  };
+  if (op.wide) return jc.u_real ? go(k_apply_packed_jac<true, EP, true>) : go(k_apply_packed_jac<false, EP, true>);
+  return jc.u_real ? go(k_apply_packed_jac<true, EP, false>) : go(k_apply_packed_jac<false, EP, false>);
 }
 
 hipError_t launch_apply_packed_jac(const DevPacked& op, const DevJacobi& jc, const double* x, double* y, bool rdo,
                                    hipStream_t s) {
   if (!apply_jac_fusable(op, jc) || (rdo && op.trace_slot < 0)) return hipErrorInvalidValue;
   const int64_t blocks = apply_jac_blocks(op);
-  const TfqEpi none{};
-  if (jc.u_real)
-    hipLaunchKernelGGL((k_apply_packed_jac<true, 0>), dim3((unsigned)blocks), dim3(256), 0, s, op, jc, x, y,
-                       rdo ? 1 : 0, none);
-  else
-    hipLaunchKernelGGL((k_apply_packed_jac<false, 0>), dim3((unsigned)blocks), dim3(256), 0, s, op, jc, x, y,
-                       rdo ? 1 : 0, none);
-  return hipGetLastError();
+  return launch_jac<0>(op, jc, x, y, rdo, TfqEpi{}, blocks, s);
 }
 
 int64_t apply_jac_blocks(const DevPacked& op) { return op.n_heavy + op.n_lt_blocks; }
@@ -1753,16 +1921,8 @@ hipError_t launch_apply_packed_jac_tfq(const DevPacked& op, const DevJacobi& jc,
   if (!apply_jac_fusable(op, jc) || (rdo && op.trace_slot < 0) || (kind != 1 && kind != 2) || !ep.s ||
       !ep.partial || (kind == 1 && !ep.w) || (kind == 2 && (!ep.prev || !ep.prev_out)))
     return hipErrorInvalidValue;
-  const dim3 grid((unsigned)apply_jac_blocks(op));
-  const int r = rdo ? 1 : 0;
-  if (jc.u_real) {
-    if (kind == 1) hipLaunchKernelGGL((k_apply_packed_jac<true, 1>), grid, dim3(256), 0, s, op, jc, x, y, r, ep);
-    else hipLaunchKernelGGL((k_apply_packed_jac<true, 2>), grid, dim3(256), 0, s, op, jc, x, y, r, ep);
-  } else {
-    if (kind == 1) hipLaunchKernelGGL((k_apply_packed_jac<false, 1>), grid, dim3(256), 0, s, op, jc, x, y, r, ep);
-    else hipLaunchKernelGGL((k_apply_packed_jac<false, 2>), grid, dim3(256), 0, s, op, jc, x, y, r, ep);
-  }
-  return hipGetLastError();
+  return kind == 1 ? launch_jac<1>(op, jc, x, y, rdo, ep, apply_jac_blocks(op), s)
+                   : launch_jac<2>(op, jc, x, y, rdo, ep, apply_jac_blocks(op), s);
 }
 
 hipError_t launch_jacobi_1k(const DevPacked& op, const DevJacobi& jc, const double* in, double* out, bool accumulate,
