@@ -182,8 +182,9 @@ int batch_build(const heomq_params* params, int nprob, int device, bool workspac
   HIPCHECK(upload(B->hq_union, hq));
   HIPCHECK(upload(B->hc_all, hc));
   const int64_t nrec = (int64_t)rec.size();
-  // the apply form (work granularity) timed on this shape and GPU
-  if (int rc = heomq_ctx_autotune(c, 10, nullptr, nullptr)) return rc;
+  // the context's own form (build_packed's rule): timing every form on every
+  // shape kept a mixture of forms whose times differ by less than the timing's
+  // noise, and the multi-shape launch then needs the kernel of every form
   B->bf = c->pfwd;
   B->bf.rec = B->rec_all.as<DevRec>();
   B->bf.gam = B->gam_all.as<double>();

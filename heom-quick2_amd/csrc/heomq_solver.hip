@@ -102,6 +102,20 @@ struct MultiLoc {
 #define SPAN_LOOP(i, sp) \
   for (int64_t i = (sp).blk * blockDim.x + threadIdx.x; i < (sp).n2; i += (sp).nblk * blockDim.x)
 
+// The iteration's vector kernels (k_step1, k_step2, k_v) load their first
+// elements, and the partial sums they fold, before they look at the scalars,
+// and each next element before the current one is written.  On the single
+// impurity a thread has one element, so a kernel's time is its chain of loads:
+// scalars, partial sums and elements one after another took k_step2 and k_v
+// 9.0 and 8.8 us at 37,012 elements (3 us of vector traffic is not the bound).
+template <typename V>
+__device__ inline V ld_if(const V* p, int64_t i, bool on) {
+  V z;
+  z.x = 0;
+  z.y = 0;
+  return on ? p[i] : z;
+}
+
 // Phase 1 of a span's reduction: the block's (a, b) partial sums in its slot.
 __device__ inline void span_partial(double a, double b, double* partial, const Span& sp) {
   block_sum2(a, b);
@@ -114,14 +128,18 @@ __device__ inline void span_partial(double a, double b, double* partial, const S
 // A reduction's phase 2 folded into the kernel that consumes it: every
 // workgroup sums its problem's partial sums (nblk pairs) in the order of
 // k_finalize's 256-thread fold, so every workgroup (and the separate
-// finalize it replaces) gets the same bits.  Every thread receives (a, b).
-__device__ inline void fold_partials(const double* __restrict__ partial, int64_t nblk, double& a, double& b) {
-  __shared__ double fa, fb;
-  double x = 0, y = 0;
+// finalize it replaces) gets the same bits.  fold_load issues the thread's
+// loads; fold_sum's result reaches every thread.
+__device__ inline void fold_load(const double* __restrict__ partial, int64_t nblk, double& x, double& y) {
+  x = 0;
+  y = 0;
   for (int64_t t = threadIdx.x; t < nblk; t += blockDim.x) {
     x += partial[2 * t];
     y += partial[2 * t + 1];
   }
+}
+__device__ inline void fold_sum(double x, double y, double& a, double& b) {
+  __shared__ double fa, fb;
   block_sum2(x, y);
   if (threadIdx.x == 0) {
     fa = x;
@@ -134,13 +152,39 @@ __device__ inline void fold_partials(const double* __restrict__ partial, int64_t
 
 
 // One quasi-minimisation half step from ||w||^2 = a.
-__device__ inline void half_step(TfqmrScal* s, double a) {
-  const double theta = sqrt(a) / s->tau;
-  const double c = 1.0 / sqrt(1.0 + theta * theta);
-  s->tau = s->tau * theta * c;
-  s->theta = theta;
-  s->eta = c * c * s->alpha;
-  s->dcoef = theta * theta * s->eta / s->alpha;
+struct Half {
+  double theta, tau, eta, dcoef;
+};
+__device__ inline Half half_of(double a, double tau, double alpha) {
+  Half h;
+  h.theta = sqrt(a) / tau;
+  const double c = 1.0 / sqrt(1.0 + h.theta * h.theta);
+  h.tau = tau * h.theta * c;
+  h.eta = c * c * alpha;
+  h.dcoef = h.theta * h.theta * h.eta / alpha;
+  return h;
+}
+__device__ inline void put_half(TfqmrScal* s, const Half& h) {
+  s->theta = h.theta;
+  s->tau = h.tau;
+  s->eta = h.eta;
+  s->dcoef = h.dcoef;
+}
+__device__ inline void half_step(TfqmrScal* s, double a) { put_half(s, half_of(a, s->tau, s->alpha)); }
+
+// The scalars copied word by word through registers.  (A TfqmrScal local to
+// k_step2 or k_v, read and written through its address, was given 69 and 32 KB
+// of LDS per workgroup, two and four workgroups per CU.)
+__device__ inline void copy_scal(const TfqmrScal* from, TfqmrScal* to) {
+  constexpr int kWords = sizeof(TfqmrScal) / 8;
+  static_assert(sizeof(TfqmrScal) % 8 == 0, "TfqmrScal is whole 8-byte words");
+  const double* p = reinterpret_cast<const double*>(from);
+  double* q = reinterpret_cast<double*>(to);
+  double v[kWords];
+#pragma unroll
+  for (int k = 0; k < kWords; ++k) v[k] = p[k];
+#pragma unroll
+  for (int k = 0; k < kWords; ++k) q[k] = v[k];
 }
 
 // The second half step of an iteration, then rho_new = rt.w = b: the bound
@@ -232,34 +276,42 @@ __global__ void k_step1(const Loc loc, T* __restrict__ w, T* __restrict__ y2, co
   using V = typename W2<T>::type;
   const Span sp = loc.span();
   s += sp.q;
-  if (s->flag) return;
   { const int64_t o = sp.off; w += o; y2 += o; v += o; aw += o; u2 += o; d += o; }
+  const int64_t step = sp.nblk * blockDim.x;
+  int64_t i = sp.blk * blockDim.x + threadIdx.x;
+  V wi, yo, a, u, b, di;
+  auto load = [&](int64_t k) {
+    const bool on = k < sp.n2;
+    wi = ld_if(reinterpret_cast<const V*>(w), k, on);
+    yo = ld_if(reinterpret_cast<const V*>(y2), k, on);
+    a = ld_if(reinterpret_cast<const V*>(aw), k, on);
+    u = ld_if(reinterpret_cast<const V*>(u2), k, on);
+    b = ld_if(reinterpret_cast<const V*>(v), k, on);
+    di = ld_if(reinterpret_cast<const V*>(d), k, on);
+  };
+  load(i);
+  if (s->flag) return;
   const T alpha = (T)s->alpha, dcoef = (T)s->dcoef, beta = (T)s->beta;
   double ww = 0;
-  SPAN_LOOP(i, sp) {
-    V wi = reinterpret_cast<V*>(w)[i];
-    const V yo = reinterpret_cast<const V*>(y2)[i];
-    V y1;
+  while (i < sp.n2) {
+    V y1, u1, o, wn, dn;
     y1.x = wi.x + beta * yo.x;
     y1.y = wi.y + beta * yo.y;
-    const V a = reinterpret_cast<const V*>(aw)[i], u = reinterpret_cast<const V*>(u2)[i];
-    V u1;
     u1.x = a.x + beta * u.x;
     u1.y = a.y + beta * u.y;
-    const V b = reinterpret_cast<const V*>(v)[i];
-    V o;
     o.x = y1.x - alpha * b.x;
     o.y = y1.y - alpha * b.y;
-    reinterpret_cast<V*>(y2)[i] = o;
-    wi.x -= alpha * u1.x;
-    wi.y -= alpha * u1.y;
-    reinterpret_cast<V*>(w)[i] = wi;
-    const V di = reinterpret_cast<const V*>(d)[i];
-    V dn;
+    wn.x = wi.x - alpha * u1.x;
+    wn.y = wi.y - alpha * u1.y;
     dn.x = y1.x + dcoef * di.x;
     dn.y = y1.y + dcoef * di.y;
-    reinterpret_cast<V*>(d)[i] = dn;
-    ww += (double)wi.x * wi.x + (double)wi.y * wi.y;
+    ww += (double)wn.x * wn.x + (double)wn.y * wn.y;
+    const int64_t at = i;
+    i += step;
+    load(i);
+    reinterpret_cast<V*>(y2)[at] = o;
+    reinterpret_cast<V*>(w)[at] = wn;
+    reinterpret_cast<V*>(d)[at] = dn;
   }
   span_partial(ww, 0.0, partial, sp);
 }
@@ -278,37 +330,48 @@ __global__ void k_step2(const Loc loc, T* __restrict__ x, T* __restrict__ w, con
   const Span sp = loc.span();
   s += sp.q;
   s_out += sp.q;
-  TfqmrScal t = *s;
-  if (t.flag) {   // uniform over the problem's workgroups
-    if (sp.blk == 0 && threadIdx.x == 0) *s_out = t;
-    return;
-  }
-  double a, unused;
-  fold_partials(part_in + 2 * (sp.pidx - sp.blk), sp.nblk, a, unused);
-  half_step(&t, a);
-  if (sp.blk == 0 && threadIdx.x == 0) *s_out = t;
-  const uint64_t seed = t.seed;
   { const int64_t o = sp.off; x += o; w += o; u2 += o; d += o; y2 += o; }
-  const T alpha = (T)t.alpha, dcoef = (T)t.dcoef, eta = (T)t.eta;
+  const int64_t step = sp.nblk * blockDim.x;
+  int64_t i = sp.blk * blockDim.x + threadIdx.x;
+  V di, xi, wi, ui, yi;
+  auto load = [&](int64_t k) {
+    const bool on = k < sp.n2;
+    di = ld_if(reinterpret_cast<const V*>(d), k, on);
+    xi = ld_if(reinterpret_cast<const V*>(x), k, on);
+    wi = ld_if(reinterpret_cast<const V*>(w), k, on);
+    ui = ld_if(reinterpret_cast<const V*>(u2), k, on);
+    yi = ld_if(reinterpret_cast<const V*>(y2), k, on);
+  };
+  double pa, pb;
+  fold_load(part_in + 2 * (sp.pidx - sp.blk), sp.nblk, pa, pb);
+  load(i);
+  const double tau = s->tau, alpha0 = s->alpha;
+  const uint64_t seed = s->seed;
+  const bool first = sp.blk == 0 && threadIdx.x == 0;
+  if (first) copy_scal(s, s_out);
+  if (s->flag) return;   // uniform over the problem's workgroups
+  double a, unused;
+  fold_sum(pa, pb, a, unused);
+  const Half h = half_of(a, tau, alpha0);
+  if (first) put_half(s_out, h);
+  const T alpha = (T)alpha0, dcoef = (T)h.dcoef, eta = (T)h.eta;
   double ww = 0, rw = 0;
-  SPAN_LOOP(i, sp) {
-    const V di = reinterpret_cast<const V*>(d)[i];
-    V xi = reinterpret_cast<V*>(x)[i];
-    xi.x += eta * di.x;
-    xi.y += eta * di.y;
-    reinterpret_cast<V*>(x)[i] = xi;
-    V wi = reinterpret_cast<V*>(w)[i];
-    const V ui = reinterpret_cast<const V*>(u2)[i];
-    wi.x -= alpha * ui.x;
-    wi.y -= alpha * ui.y;
-    reinterpret_cast<V*>(w)[i] = wi;
-    const V yi = reinterpret_cast<const V*>(y2)[i];
-    V dn;
+  while (i < sp.n2) {
+    V xn, wn, dn;
+    xn.x = xi.x + eta * di.x;
+    xn.y = xi.y + eta * di.y;
+    wn.x = wi.x - alpha * ui.x;
+    wn.y = wi.y - alpha * ui.y;
     dn.x = yi.x + dcoef * di.x;
     dn.y = yi.y + dcoef * di.y;
-    reinterpret_cast<V*>(d)[i] = dn;
-    ww += (double)wi.x * wi.x + (double)wi.y * wi.y;
-    rw += shadow(2 * i, seed) * wi.x + shadow(2 * i + 1, seed) * wi.y;
+    ww += (double)wn.x * wn.x + (double)wn.y * wn.y;
+    rw += shadow(2 * i, seed) * wn.x + shadow(2 * i + 1, seed) * wn.y;
+    const int64_t at = i;
+    i += step;
+    load(i);
+    reinterpret_cast<V*>(x)[at] = xn;
+    reinterpret_cast<V*>(w)[at] = wn;
+    reinterpret_cast<V*>(d)[at] = dn;
   }
   span_partial(ww, rw, partial, sp);
 }
@@ -327,32 +390,60 @@ __global__ void k_v(const Loc loc, const T* __restrict__ aw, const T* __restrict
   const Span sp = loc.span();
   s_in += sp.q;
   s_out += sp.q;
-  TfqmrScal t = *s_in;
-  if (t.flag) return;   // s_out already holds this state
-  double a, b;
-  fold_partials(part_in + 2 * (sp.pidx - sp.blk), sp.nblk, a, b);
-  half_step_rho(&t, a, b);
-  if (sp.blk == 0 && threadIdx.x == 0) *s_out = t;
-  if (t.flag) return;   // breakdown: no update (uniform over the problem's workgroups)
-  const uint64_t seed = t.seed;
   { const int64_t o = sp.off; aw += o; u2 += o; v += o; x += o; d += o; }
-  const T beta = (T)t.beta, eta = (T)t.eta;
-  const bool next = t.stop == 0;
+  const int64_t step = sp.nblk * blockDim.x;
+  int64_t i = sp.blk * blockDim.x + threadIdx.x;
+  V xi, di, a2, b2, c;
+  auto load = [&](int64_t k) {
+    const bool on = k < sp.n2;
+    xi = ld_if(reinterpret_cast<const V*>(x), k, on);
+    di = ld_if(reinterpret_cast<const V*>(d), k, on);
+    a2 = ld_if(reinterpret_cast<const V*>(aw), k, on);
+    b2 = ld_if(reinterpret_cast<const V*>(u2), k, on);
+    c = ld_if(reinterpret_cast<const V*>(v), k, on);
+  };
+  double pa, pb;
+  fold_load(part_in + 2 * (sp.pidx - sp.blk), sp.nblk, pa, pb);
+  load(i);
+  const double tau = s_in->tau, alpha0 = s_in->alpha, rho = s_in->rho, target = s_in->target, beta0 = s_in->beta;
+  const int iter = s_in->iter + 1;
+  const uint64_t seed = s_in->seed;
+  if (s_in->flag) return;   // s_out already holds this state
+  const bool first = sp.blk == 0 && threadIdx.x == 0;
+  if (first) copy_scal(s_in, s_out);
+  double a, b;
+  fold_sum(pa, pb, a, b);
+  // half_step_rho on values
+  const Half h = half_of(a, tau, alpha0);
+  const bool next = !(h.tau * sqrt(2.0 * iter + 1.0) <= target);
+  const bool broken = next && rho == 0.0;
+  const double beta1 = next && !broken ? b / rho : beta0;
+  if (first) {
+    put_half(s_out, h);
+    s_out->iter = iter;
+    if (!next) s_out->stop = 1;
+    if (broken) s_out->flag = 2;
+    if (next && !broken) {
+      s_out->beta = beta1;
+      s_out->rho = b;
+    }
+  }
+  if (broken) return;   // no update (uniform over the problem's workgroups)
+  const T beta = (T)beta1, eta = (T)h.eta;
   double sg = 0;
-  SPAN_LOOP(i, sp) {
-    V xi = reinterpret_cast<V*>(x)[i];
-    const V di = reinterpret_cast<const V*>(d)[i];
-    xi.x += eta * di.x;
-    xi.y += eta * di.y;
-    reinterpret_cast<V*>(x)[i] = xi;
+  while (i < sp.n2) {
+    V xn, r;
+    xn.x = xi.x + eta * di.x;
+    xn.y = xi.y + eta * di.y;
+    r.x = a2.x + beta * ((T)2 * b2.x + beta * c.x);
+    r.y = a2.y + beta * ((T)2 * b2.y + beta * c.y);
+    const int64_t at = i;
+    i += step;
+    load(i);
+    reinterpret_cast<V*>(x)[at] = xn;
     if (next) {
-      const V a2 = reinterpret_cast<const V*>(aw)[i], b2 = reinterpret_cast<const V*>(u2)[i];
-      const V c = reinterpret_cast<const V*>(v)[i];
-      V r;
-      r.x = a2.x + beta * ((T)2 * b2.x + beta * c.x);
-      r.y = a2.y + beta * ((T)2 * b2.y + beta * c.y);
-      reinterpret_cast<V*>(v)[i] = r;
-      sg += shadow(2 * i, seed) * r.x + shadow(2 * i + 1, seed) * r.y;
+      reinterpret_cast<V*>(v)[at] = r;
+      sg += shadow(2 * at, seed) * r.x + shadow(2 * at + 1, seed) * r.y;
     }
   }
   span_partial(sg, 0.0, partial, sp);

@@ -517,7 +517,7 @@ int heomq_batch_solve(heomq_batch* b, double tol, int maxiter, double* rdo, doub
  * grouped by shape (each shape's structural tables shared, as a batch), and
  * every packed apply and every TFQMR vector kernel runs over a flat grid that
  * covers every problem of every shape, largest shape first; each shape's
- * apply form is the one heomq_ctx_autotune picks for it.  Each problem keeps the blocks-per-problem count of a solve
+ * apply form is a context's default for it.  Each problem keeps the blocks-per-problem count of a solve
  * on its own, so its reductions fold the same partial sums in the same order.
  * The reference's counterpart is one process per point
  * (tools/make_input_ivcurve/ivcurve.csh); no entry point of its own.
