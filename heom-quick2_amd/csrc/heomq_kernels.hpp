@@ -360,6 +360,11 @@ struct TfqEpi {
   const double* prev = nullptr;   // kind 2: kind 1's three arrays, summed in runs of 16 into prev_out
   double* prev_out = nullptr;
 };
+// The same vector work carried by the plain apply (Jacobi-scaled when
+// op.precond is set), forward or transposed, over apply_blocks(op) workgroups.
+bool apply_tfq_fusable(const DevPacked& op);
+hipError_t launch_apply_packed_tfq(const DevPacked& op, const double* x, double* y, bool rdo, int kind,
+                                   const TfqEpi& ep, hipStream_t s);
 int64_t apply_jac_blocks(const DevPacked& op);
 hipError_t launch_apply_packed_jac_tfq(const DevPacked& op, const DevJacobi& jc, const double* x, double* y, bool rdo,
                                        int kind, const TfqEpi& ep, hipStream_t s);

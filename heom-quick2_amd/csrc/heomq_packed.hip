@@ -105,22 +105,55 @@ __device__ inline int div_by(int t, int inv) { return (int)(((uint32_t)t * (uint
 // (td/chebyshev.f90's P_k = P_{k-2} + (2 / delta) L P_{k-1} over P_{k-2},
 // then x += 2 J_k P_k), the same arithmetic as the two vector passes.
 struct ChebEpi {
+  static constexpr bool on = true, tier0 = false;
   double* p;
   double* x;
   double a, b;
+  __device__ void put(int64_t g, double re, double im) {
+    double2* pv = reinterpret_cast<double2*>(p) + g;
+    double2* xv = reinterpret_cast<double2*>(x) + g;
+    double2 q = *pv;
+    q.x += a * re;
+    q.y += a * im;
+    *pv = q;
+    double2 w = *xv;
+    w.x += b * q.x;
+    w.y += b * q.y;
+    *xv = w;
+  }
 };
-__device__ inline void cheb_put(const ChebEpi* ep, int64_t g, double re, double im) {
-  double2* pv = reinterpret_cast<double2*>(ep->p) + g;
-  double2* xv = reinterpret_cast<double2*>(ep->x) + g;
-  double2 q = *pv;
-  q.x += ep->a * re;
-  q.y += ep->a * im;
-  *pv = q;
-  double2 w = *xv;
-  w.x += ep->b * q.x;
-  w.y += ep->b * q.y;
-  *xv = w;
-}
+// No epilogue: the apply writes y.
+struct NoEpi {
+  static constexpr bool on = false, tier0 = false;
+};
+// A TFQMR iteration's vector work where the apply writes its output (one
+// problem): KIND 1, out = u2, then w -= alpha u2 and the sums ||w||^2, rt.w,
+// rt.u2 of this thread's elements; KIND 2, out = aw and rt.aw.  tier0: the
+// tier-0 block is written and fixed up first and put from memory.
+template <int KIND>
+struct TfqPut {
+  static constexpr bool on = true, tier0 = true;
+  double alpha;
+  uint64_t seed;
+  double* out;
+  double* w;
+  double r0, r1, r2;
+  __device__ void put(int64_t g, double re, double im) {
+    reinterpret_cast<double2*>(out)[g] = make_double2(re, im);
+    const double s0 = shadow(2 * g, seed), s1 = shadow(2 * g + 1, seed);
+    if (KIND == 1) {
+      double2 wi = reinterpret_cast<double2*>(w)[g];
+      wi.x -= alpha * re;
+      wi.y -= alpha * im;
+      reinterpret_cast<double2*>(w)[g] = wi;
+      r0 += wi.x * wi.x + wi.y * wi.y;
+      r1 += s0 * wi.x + s1 * wi.y;
+      r2 += s0 * re + s1 * im;
+    } else {
+      r0 += s0 * re + s1 * im;
+    }
+  }
+};
 
 // The coefficient arrays of one problem of a batch.
 struct Coefs {
@@ -350,9 +383,9 @@ constexpr size_t kHeavyOffRi = 256 * 8, kHeavyOffL = 2 * 256 * 8, kHeavyOffR = k
                  kHeavySmem = kHeavyOffX + 256 * 16;
 constexpr size_t kApplySmem0 = kLightSmem > kHeavySmem ? kLightSmem : kHeavySmem;
 
-template <typename T, bool TRANS, bool WIDE, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, class Ep = NoEpi>
 __device__ inline void light_body(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x, T* __restrict__ y,
-                                  int64_t zero_at, int bid, char* smem, bool scaled, const ChebEpi* ep = nullptr) {
+                                  int64_t zero_at, int bid, char* smem, bool scaled, Ep* ep = nullptr) {
   using V = typename P2<T>::type;
   int64_t* s_off = reinterpret_cast<int64_t*>(smem);
   int64_t* s_p0 = reinterpret_cast<int64_t*>(smem + kLightOffP0);
@@ -407,8 +440,8 @@ __device__ inline void light_body(const DevPacked& op, const Coefs cf_p, const T
     coupling_block<T, TRANS, WIDE, U>(en, cf, nv, op.maps, xs, slot, zero_at, ar, ai);
   }
   if (scaled) jacobi_scale<T>(op, (T)s_gam[l].x, (T)s_gam[l].y, csr, csi, ar, ai);
-  if (EPI) {
-    cheb_put(ep, t, (double)ar, (double)ai);
+  if constexpr (Ep::on) {
+    ep->put(t, (double)ar, (double)ai);
     return;
   }
   V o;
@@ -437,10 +470,10 @@ struct StageOut {
 // coupling of the ADO (entries and coefficients staged in LDS), two
 // couplings per step; the slices are summed through LDS in a fixed order.
 // Block 0 (the tier-0 ADO) then applies the trace row and Hermitianises.
-template <typename T, bool TRANS, bool WIDE, bool STAGE = false, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool STAGE = false, class Ep = NoEpi>
 __device__ inline void heavy_body(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x, T* __restrict__ y,
                                   int64_t zero_at, int rdo, int bid, char* smem, bool scaled,
-                                  StageOut* so = nullptr, const ChebEpi* ep = nullptr) {
+                                  StageOut* so = nullptr, Ep* ep = nullptr) {
   using V = typename P2<T>::type;
   constexpr int kStage = 256;
   T* red_r = reinterpret_cast<T*>(smem);
@@ -518,8 +551,8 @@ __device__ inline void heavy_body(const DevPacked& op, const Coefs cf_p, const T
       if (STAGE) {   // one pass (nnz <= 256): slot t = threadIdx.x
         so->v = make_double2((double)sr, (double)si);
         so->act = true;
-      } else if (EPI) {
-        cheb_put(ep, base + t, (double)sr, (double)si);
+      } else if (Ep::on && !(Ep::tier0 && a == 0)) {
+        if constexpr (Ep::on) ep->put(base + t, (double)sr, (double)si);
       } else {
         reinterpret_cast<V*>(y)[base + t] = o;
       }
@@ -533,8 +566,12 @@ __device__ inline void heavy_body(const DevPacked& op, const Coefs cf_p, const T
     so->s = s;
     so->gr = (double)gr;
     so->gi = (double)gi;
-  } else if (a == 0 && !EPI) {   // (with the epilogue no trace row and no Hermitian fix-up: host check)
+  } else if (a == 0 && (!Ep::on || Ep::tier0)) {   // (with the Chebyshev epilogue no trace row and no Hermitian fix-up: host check)
     tier0_fixup_block<T>(op, x, y, rdo);   // block-uniform branch
+    if constexpr (Ep::on) {
+      __syncthreads();
+      for (int t = threadIdx.x; t < nnz; t += 256) ep->put(base + t, (double)y[2 * (base + t)], (double)y[2 * (base + t) + 1]);
+    }
   }
 }
 
@@ -561,10 +598,10 @@ constexpr size_t kGOffB = 256 * sizeof(HWgt<double>);                           
 constexpr size_t kGOffG = kGOffB + 2 * 16 * (size_t)kHeavyPairs;                   // run table
 constexpr size_t kGSmem = kGOffG + 16 * (size_t)(kHeavyGroups + 1);
 
-template <typename T, bool TRANS, bool WIDE, bool STAGE = false, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool STAGE = false, class Ep = NoEpi>
 __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x,
                                      T* __restrict__ y, int64_t zero_at, int rdo, int bid, char* smem, bool scaled,
-                                     StageOut* so = nullptr, const ChebEpi* ep = nullptr) {
+                                     StageOut* so = nullptr, Ep* ep = nullptr) {
   using V = typename P2<T>::type;
   HWgt<T>* s_w = reinterpret_cast<HWgt<T>*>(smem);
   V* s_B = reinterpret_cast<V*>(smem + kGOffB);
@@ -696,8 +733,8 @@ __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, cons
       if (STAGE) {   // one pass (nnz <= 256): slot t = threadIdx.x
         so->v = make_double2((double)sr, (double)si);
         so->act = true;
-      } else if (EPI) {
-        cheb_put(ep, base + t, (double)sr, (double)si);
+      } else if (Ep::on && !(Ep::tier0 && a == 0)) {
+        if constexpr (Ep::on) ep->put(base + t, (double)sr, (double)si);
       } else {
         reinterpret_cast<V*>(y)[base + t] = o;
       }
@@ -711,8 +748,12 @@ __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, cons
     so->s = s;
     so->gr = (double)gr;
     so->gi = (double)gi;
-  } else if (a == 0 && !EPI) {   // (with the epilogue no trace row and no Hermitian fix-up: host check)
+  } else if (a == 0 && (!Ep::on || Ep::tier0)) {   // (with the Chebyshev epilogue no trace row and no Hermitian fix-up: host check)
     tier0_fixup_block<T>(op, x, y, rdo);   // block-uniform branch
+    if constexpr (Ep::on) {
+      __syncthreads();
+      for (int t = threadIdx.x; t < nnz; t += 256) ep->put(base + t, (double)y[2 * (base + t)], (double)y[2 * (base + t) + 1]);
+    }
   }
 }
 
@@ -722,9 +763,9 @@ __device__ inline void heavy_grouped(const DevPacked& op, const Coefs cf_p, cons
 // of two w, so 64 / w slices walk the coupling list (entries, records and
 // gather maps from global memory, two couplings in flight); the slices are
 // summed by shuffles in a fixed tree, with no LDS and no barrier.
-template <typename T, bool TRANS, bool WIDE, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, class Ep = NoEpi>
 __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x, T* __restrict__ y,
-                                  int64_t zero_at, int64_t a, bool scaled, const ChebEpi* ep = nullptr) {
+                                  int64_t zero_at, int64_t a, bool scaled, Ep* ep = nullptr) {
   using V = typename P2<T>::type;
   const int lane = threadIdx.x & 63;
   const int64_t base = op.off[a];
@@ -770,8 +811,8 @@ __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T
   }
   if (slice == 0 && act) {
     if (scaled) jacobi_scale<T>(op, gr, gi, csr, csi, ar, ai);
-    if (EPI) {
-      cheb_put(ep, base + t, (double)ar, (double)ai);
+    if constexpr (Ep::on) {
+      ep->put(base + t, (double)ar, (double)ai);
       return;
     }
     V o;
@@ -797,10 +838,10 @@ constexpr size_t kLOffHc = 0, kLOffX = kLOffHc + 256 * 16, kLOffL = kLOffX + 256
                  kLOffR = kLOffL + kLStage * 16, kLOffBm = kLOffR + kLStage * 16, kLOffG = kLOffBm + kLStage * 8,
                  kLSmem = kLOffG + kLStage * 16;
 
-template <typename T, bool TRANS, bool WIDE, bool STAGE = false, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, bool STAGE = false, class Ep = NoEpi>
 __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x,
                                     T* __restrict__ y, int64_t zero_at, int bid, char* smem, bool scaled,
-                                    StageOut* so = nullptr, const ChebEpi* ep = nullptr) {
+                                    StageOut* so = nullptr, Ep* ep = nullptr) {
   using V = typename P2<T>::type;
   double2* s_hc = reinterpret_cast<double2*>(smem + kLOffHc);
   V* s_x = reinterpret_cast<V*>(smem + kLOffX);
@@ -910,8 +951,8 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
     so->gi = (double)gi;
     return;
   }
-  if (EPI) {
-    cheb_put(ep, (int64_t)base + t, (double)ar, (double)ai);
+  if constexpr (Ep::on) {
+    ep->put((int64_t)base + t, (double)ar, (double)ai);
     return;
   }
   V o;
@@ -935,10 +976,10 @@ constexpr int kAnyForm = -1;
 static int apply_form(const DevPacked& op) {
   return (op.hg_off ? 1 : 0) | (op.lt_blk ? 2 : 0) | (op.heavy_wave ? 4 : 0);
 }
-template <typename T, bool TRANS, bool WIDE, int FORM, bool EPI = false>
+template <typename T, bool TRANS, bool WIDE, int FORM, class Ep = NoEpi>
 __device__ inline void apply_block(const DevPacked& op, int64_t p, int64_t bx, const T* __restrict__ x,
                                    T* __restrict__ y, int64_t zero_at, int rdo, char* smem,
-                                   const ChebEpi* ep = nullptr) {
+                                   Ep* ep = nullptr) {
   if (op.frozen_flag && op.frozen_flag[p * op.frozen_stride] == 3) return;   // finished: block-uniform, no barrier yet
   const bool scaled = op.precond && !(op.frozen_flag && op.frozen_flag[p * op.frozen_stride + 2]);
   x += 2 * p * op.vstride;
@@ -951,18 +992,18 @@ __device__ inline void apply_block(const DevPacked& op, int64_t p, int64_t bx, c
   if (bx < hb) {   // block-uniform
     if (wave && bx > 0) {   // four ADOs of small sectors, a wave each (no barrier)
       const int64_t a = 1 + (bx - 1) * 4 + (threadIdx.x >> 6);
-      if (a < op.n_heavy) heavy_wave<T, TRANS, WIDE, EPI>(op, cf, x, y, zero_at, a, scaled, ep);
+      if (a < op.n_heavy) heavy_wave<T, TRANS, WIDE, Ep>(op, cf, x, y, zero_at, a, scaled, ep);
       return;
     }
     const int a = (int)bx;
     if (grouped && op.hg_off[a + 1] > op.hg_off[a])
-      heavy_grouped<T, TRANS, WIDE, false, EPI>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
+      heavy_grouped<T, TRANS, WIDE, false, Ep>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
     else
-      heavy_body<T, TRANS, WIDE, false, EPI>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
+      heavy_body<T, TRANS, WIDE, false, Ep>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
   } else if (sector) {
-    light_sector<T, TRANS, WIDE, false, EPI>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, nullptr, ep);
+    light_sector<T, TRANS, WIDE, false, Ep>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, nullptr, ep);
   } else {
-    light_body<T, TRANS, WIDE, EPI>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, ep);
+    light_body<T, TRANS, WIDE, Ep>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, ep);
   }
 }
 
@@ -980,7 +1021,8 @@ template <bool WIDE, int FORM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 k_apply_packed_cheb(const DevPacked op, const double* __restrict__ p1, const ChebEpi ep) {
   __shared__ __align__(16) char smem[kApplySmem];
-  apply_block<double, false, WIDE, FORM, true>(op, 0, blockIdx.x, p1, nullptr, -1, 0, smem, &ep);
+  ChebEpi e = ep;
+  apply_block<double, false, WIDE, FORM, ChebEpi>(op, 0, blockIdx.x, p1, nullptr, -1, 0, smem, &e);
 }
 
 // Forward applies of problems of several shapes in one flat grid (the shapes
@@ -1447,6 +1489,67 @@ __global__ __launch_bounds__(256) void k_jacobi_ado(const DevPacked op, const De
   xo[w0 + tid] = o;
 }
 
+// The sums of a TFQMR epilogue over the workgroup into its partial slots (EP 1:
+// three, EP 2: one and the first launch's sums added up in runs of 16
+// workgroups, for the fold).
+template <int EP>
+__device__ inline void tfq_partials(double r0, double r1, double r2, const TfqEpi& ep) {
+  const int tid = threadIdx.x;
+  __shared__ double red[3][4];
+  for (int off = 32; off > 0; off >>= 1) {
+    r0 += __shfl_down(r0, off, 64);
+    if (EP == 1) {
+      r1 += __shfl_down(r1, off, 64);
+      r2 += __shfl_down(r2, off, 64);
+    }
+  }
+  const int lane = tid & 63, wid = tid >> 6;
+  if (lane == 0) {
+    red[0][wid] = r0;
+    red[1][wid] = r1;
+    red[2][wid] = r2;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    double a = 0, b = 0, c = 0;
+    for (int k = 0; k < 4; ++k) {
+      a += red[0][k];
+      b += red[1][k];
+      c += red[2][k];
+    }
+    if (EP == 1) {
+      ep.partial[blockIdx.x] = a;
+      ep.partial[gridDim.x + blockIdx.x] = b;
+      ep.partial[2 * gridDim.x + blockIdx.x] = c;
+    } else {
+      ep.partial[blockIdx.x] = a;
+    }
+  }
+  if (EP == 2) {   // the first launch's sums, 16 workgroups' worth per workgroup here, for the fold
+    const int na = (int)gridDim.x, ng = (na + 15) >> 4;
+    if ((int)blockIdx.x < ng && tid < 64) {   // wave 0: lanes (k, j), k = tid / 16 < 3 the sum
+      const int k = tid >> 4, j = tid & 15, idx = (int)blockIdx.x * 16 + j;
+      double v = (k < 3 && idx < na) ? ep.prev[(int64_t)k * na + idx] : 0.0;
+      for (int off = 8; off > 0; off >>= 1) v += __shfl_down(v, off, 16);
+      if (k < 3 && j == 0) ep.prev_out[(int64_t)k * ng + blockIdx.x] = v;
+    }
+  }
+}
+
+// The plain (or Jacobi-scaled) apply with a TFQMR iteration's vector work on
+// its outputs (TfqPut): k_step2 and the v update of k_v and their launches are
+// gone from the iteration, as in the preconditioned one below.
+template <bool TRANS, int FORM, int KIND>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
+k_apply_packed_tfq(const DevPacked op, const double* __restrict__ x, double* __restrict__ y, int64_t zero_at, int rdo,
+                   const TfqEpi ep) {
+  if (ep.s->flag) return;   // uniform over the grid
+  __shared__ __align__(16) char smem[kApplySmem];
+  TfqPut<KIND> e{ep.s->alpha, ep.s->seed, y, ep.w, 0.0, 0.0, 0.0};
+  apply_block<double, TRANS, false, FORM, TfqPut<KIND>>(op, 0, blockIdx.x, x, y, zero_at, rdo, smem, &e);
+  tfq_partials<KIND>(e.r0, e.r1, e.r2, ep);
+}
+
 // The block-Jacobi-preconditioned apply in one launch, y = M^-1 (Pi A x):
 // each workgroup of the apply holds whole ADOs (a heavy ADO, or a
 // sector-batched run of top-tier ADOs), so it keeps its outputs in registers,
@@ -1613,45 +1716,7 @@ k_apply_packed_jac(const DevPacked op, const DevJacobi jc, const double* __restr
       r0 = s0 * z.x + s1 * z.y;
     }
   }
-  __shared__ double red[3][4];
-  for (int off = 32; off > 0; off >>= 1) {
-    r0 += __shfl_down(r0, off, 64);
-    if (EP == 1) {
-      r1 += __shfl_down(r1, off, 64);
-      r2 += __shfl_down(r2, off, 64);
-    }
-  }
-  const int lane = tid & 63, wid = tid >> 6;
-  if (lane == 0) {
-    red[0][wid] = r0;
-    red[1][wid] = r1;
-    red[2][wid] = r2;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    double a = 0, b = 0, c = 0;
-    for (int k = 0; k < 4; ++k) {
-      a += red[0][k];
-      b += red[1][k];
-      c += red[2][k];
-    }
-    if (EP == 1) {
-      ep.partial[blockIdx.x] = a;
-      ep.partial[gridDim.x + blockIdx.x] = b;
-      ep.partial[2 * gridDim.x + blockIdx.x] = c;
-    } else {
-      ep.partial[blockIdx.x] = a;
-    }
-  }
-  if (EP == 2) {   // the first launch's sums, 16 workgroups' worth per workgroup here, for the fold
-    const int na = (int)gridDim.x, ng = (na + 15) >> 4;
-    if ((int)blockIdx.x < ng && tid < 64) {   // wave 0: lanes (k, j), k = tid / 16 < 3 the sum
-      const int k = tid >> 4, j = tid & 15, idx = (int)blockIdx.x * 16 + j;
-      double v = (k < 3 && idx < na) ? ep.prev[(int64_t)k * na + idx] : 0.0;
-      for (int off = 8; off > 0; off >>= 1) v += __shfl_down(v, off, 16);
-      if (k < 3 && j == 0) ep.prev_out[(int64_t)k * ng + blockIdx.x] = v;
-    }
-  }
+  tfq_partials<EP>(r0, r1, r2, ep);
 }
 
 template <typename TP, typename TD>
@@ -1912,6 +1977,32 @@ hipError_t launch_apply_packed_jac(const DevPacked& op, const DevJacobi& jc, con
   if (!apply_jac_fusable(op, jc) || (rdo && op.trace_slot < 0)) return hipErrorInvalidValue;
   const int64_t blocks = apply_jac_blocks(op);
   return launch_jac<0>(op, jc, x, y, rdo, TfqEpi{}, blocks, s);
+}
+
+bool apply_tfq_fusable(const DevPacked& op) {
+  return op.nprob == 1 && !op.wide && op.n_heavy > 0 && op.frozen_flag == nullptr && apply_blocks(op) > 0;
+}
+
+hipError_t launch_apply_packed_tfq(const DevPacked& op, const double* x, double* y, bool rdo, int kind,
+                                   const TfqEpi& ep, hipStream_t s) {
+  if (!apply_tfq_fusable(op) || (rdo && op.trace_slot < 0) || (kind != 1 && kind != 2) || !ep.s || !ep.partial ||
+      (kind == 1 && !ep.w) || (kind == 2 && (!ep.prev || !ep.prev_out)))
+    return hipErrorInvalidValue;
+  const int64_t zero_at = (op.transposed && rdo) ? op.trace_slot : -1;
+  const dim3 grid((unsigned)apply_blocks(op));
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, op, x, y, zero_at, rdo ? 1 : 0, ep);
+    return hipGetLastError();
+  };
+  auto pick = [&](auto trans, auto k) {
+    constexpr bool TR = decltype(trans)::value;
+    constexpr int K = decltype(k)::value;
+    return apply_form(op) == 6 ? go(k_apply_packed_tfq<TR, 6, K>) : go(k_apply_packed_tfq<TR, kAnyForm, K>);
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  if (op.transposed) return kind == 1 ? pick(std::true_type{}, One{}) : pick(std::true_type{}, Two{});
+  return kind == 1 ? pick(std::false_type{}, One{}) : pick(std::false_type{}, Two{});
 }
 
 int64_t apply_jac_blocks(const DevPacked& op) { return op.n_heavy + op.n_lt_blocks; }

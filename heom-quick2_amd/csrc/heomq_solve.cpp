@@ -132,19 +132,27 @@ struct RunStats {
   bool fused = false;   // some iterations ran with their vector work in the operator launches
 };
 
-// Whether the block-Jacobi iteration can run with its vector work carried by
-// the fused preconditioned launches (FP64, forward operator, one problem);
+// The operator a fused iteration launches: the packed operator, Jacobi-scaled
+// for prec 1.
+DevPacked fused_operator(heomq_ctx* c, bool trans, int prec) {
+  DevPacked op = trans ? c->ptrn : c->pfwd;
+  op.precond = prec == 1 ? 1 : 0;
+  return op;
+}
+
+// Whether the iteration can run with its vector work carried by the operator
+// launches (FP64, one problem): block Jacobi (prec 2) by the fused
+// preconditioned launches, the plain or Jacobi-scaled operator by its own;
 // HEOMQ_TFQ_FUSED=0 keeps the five-kernel iteration for comparison.
-bool tfq_fusable(heomq_ctx* c, bool trans, bool rdo) {
+bool tfq_fusable(heomq_ctx* c, bool trans, bool rdo, int prec) {
   static const bool off = [] {
     const char* e = std::getenv("HEOMQ_TFQ_FUSED");
     return e && e[0] == '0';
   }();
-  if (off || trans || !c->fuse_precond || c->trun.built) return false;
-  DevPacked op = c->pfwd;
-  op.precond = 0;
-  DevJacobi jc = c->pjac;
-  return apply_jac_fusable(op, jc) && (!rdo || op.trace_slot >= 0);
+  if (off || !c->fuse_precond || c->trun.built) return false;
+  const DevPacked op = fused_operator(c, trans, prec);
+  if (rdo && op.trace_slot < 0) return false;
+  return prec == 2 ? !trans && apply_jac_fusable(op, c->pjac) : apply_tfq_fusable(op);
 }
 
 // Sums of the fused iteration's operator launches over na workgroups: four
@@ -155,22 +163,23 @@ size_t tfq_fused_sums(int64_t na) { return 4 * (size_t)na + 3 * (size_t)((na + 1
 // deferred x, d and v work), M^-1 A y2 with step 2, M^-1 A w with the rt.aw
 // sums, and the one-block fold of all three reductions.
 hipError_t record_fused(heomq_ctx* c, double* x, const Work<double>& W, int64_t n, hipStream_t st, bool rdo,
-                        int iters) {
+                        int iters, bool trans, int prec) {
   TfqmrScal* s = c->scal.as<TfqmrScal>();
   double* part = c->partial.as<double>();
-  DevPacked op = c->pfwd;
-  op.precond = 0;
+  const DevPacked op = fused_operator(c, trans, prec);
   DevJacobi jc = c->pjac;
   jc.ejac = c->prec_shift;
-  const int na = (int)apply_jac_blocks(op);
+  const int na = (int)(prec == 2 ? apply_jac_blocks(op) : apply_blocks(op));
   double* pa = c->partial_apply.as<double>();
   if (!pa || c->partial_apply.bytes < sizeof(double) * tfq_fused_sums(na)) return hipErrorInvalidValue;
+  auto apply = [&](const double* in, double* out, int kind, const TfqEpi& ep) {
+    return prec == 2 ? launch_apply_packed_jac_tfq(op, jc, in, out, rdo, kind, ep, st)
+                     : launch_apply_packed_tfq(op, in, out, rdo, kind, ep, st);
+  };
   for (int k = 0; k < iters; ++k) {
     if (hipError_t e = tfq_step1_fused(st, n, W.w, W.y2, W.v, W.aw, W.u2, W.d, x, s, part)) return e;
-    if (hipError_t e = launch_apply_packed_jac_tfq(op, jc, W.y2, W.u2, rdo, 1, TfqEpi{s, W.w, pa}, st)) return e;
-    if (hipError_t e = launch_apply_packed_jac_tfq(op, jc, W.w, W.aw, rdo, 2,
-                                                   TfqEpi{s, nullptr, pa + 3 * na, pa, pa + 4 * na}, st))
-      return e;
+    if (hipError_t e = apply(W.y2, W.u2, 1, TfqEpi{s, W.w, pa})) return e;
+    if (hipError_t e = apply(W.w, W.aw, 2, TfqEpi{s, nullptr, pa + 3 * na, pa, pa + 4 * na})) return e;
     if (hipError_t e = tfq_fold(st, n, part, pa, na, s)) return e;
   }
   return hipSuccess;
@@ -180,9 +189,9 @@ hipError_t record_fused(heomq_ctx* c, double* x, const Work<double>& W, int64_t 
 // the fused iteration, with the trace row when fused is 1).
 template <typename T, typename Apply>
 hipError_t record_chunk(heomq_ctx* c, T* x, const Work<T>& W, int64_t n, hipStream_t st, Apply& A, int iters,
-                        int fused = -1) {
+                        int fused = -1, bool trans = false, int prec = 0) {
   if (fused >= 0) {
-    if constexpr (std::is_same<T, double>::value) return record_fused(c, x, W, n, st, fused == 1, iters);
+    if constexpr (std::is_same<T, double>::value) return record_fused(c, x, W, n, st, fused == 1, iters, trans, prec);
     return hipErrorInvalidValue;
   }
   TfqmrScal* s = c->scal.as<TfqmrScal>();
@@ -205,7 +214,7 @@ hipError_t record_chunk(heomq_ctx* c, T* x, const Work<T>& W, int64_t n, hipStre
 // convergence or breakdown does nothing.
 template <typename T, typename Apply>
 int chunk_graph(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool trans, int64_t tpos, int mode,
-                hipStream_t st, Apply& A, int iters, hipGraphExec_t* out, int fused = -1) {
+                hipStream_t st, Apply& A, int iters, hipGraphExec_t* out, int fused = -1, int prec = 0) {
   for (const auto& g : c->graphs)
     if (g.x == x && g.b == b && g.work == W.w && g.n == n && g.tpos == tpos && g.mode == mode &&
         g.trans == (int)trans && g.bytes == (int)sizeof(T) && g.stream == st) {
@@ -215,7 +224,7 @@ int chunk_graph(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, boo
   if (std::getenv("HEOMQ_SOLVER_LOG"))
     std::fprintf(stderr, "tfqmr: capturing a chunk graph (mode %d, %zu cached)\n", mode, c->graphs.size());
   HIPCHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  const hipError_t rec = record_chunk<T>(c, x, W, n, st, A, iters, fused);
+  const hipError_t rec = record_chunk<T>(c, x, W, n, st, A, iters, fused, trans, prec);
   hipGraph_t graph = nullptr;
   const hipError_t end = hipStreamEndCapture(st, &graph);
   if (rec != hipSuccess || end != hipSuccess) {
@@ -262,11 +271,14 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
     HIPCHECK(precond_rhs(c, b, W.bp, W.pt, st));
   }
   if (prec == 1 && W.bp) HIPCHECK(launch_jacobi_scale_rhs<T>(trans ? c->ptrn : c->pfwd, b, W.bp, st));
-  bool fuse_ok = false;
-  if constexpr (std::is_same<T, double>::value) fuse_ok = mode == 1 && prec == 2 && tfq_fusable(c, trans, tpos >= 0);
-  if (fuse_ok) {   // captured chunks hold the buffer's address: a new buffer retires them
+  auto fuse_ok = [&]() -> bool {   // for the current preconditioner (a stalled one is dropped)
+    if constexpr (std::is_same<T, double>::value) return mode == 1 && tfq_fusable(c, trans, tpos >= 0, prec);
+    return false;
+  };
+  if (fuse_ok()) {   // captured chunks hold the buffer's address: a new buffer retires them
+    const DevPacked op = fused_operator(c, trans, prec);
     const void* before = c->partial_apply.p;
-    HIPCHECK(c->partial_apply.alloc(sizeof(double) * tfq_fused_sums(apply_jac_blocks(c->pfwd))));
+    HIPCHECK(c->partial_apply.alloc(sizeof(double) * tfq_fused_sums(std::max(apply_jac_blocks(op), apply_blocks(op)))));
     if (c->partial_apply.p != before) c->drop_graphs();
   }
   TfqmrScal* s = c->scal.as<TfqmrScal>();
@@ -335,7 +347,7 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
     int no_progress = 0;
     double last_check = rr;
     // the fused iteration leaves x one deferred update behind: flush() before x is read
-    const int fused = (prec == 2 && fuse_ok) ? (tpos >= 0 ? 1 : 0) : -1;
+    const int fused = fuse_ok() && c->partial_apply.p ? (tpos >= 0 ? 1 : 0) : -1;
     rs.fused = rs.fused || fused >= 0;
     auto flush = [&]() -> hipError_t {
       if constexpr (std::is_same<T, double>::value)
@@ -344,13 +356,13 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
     };
     if (c->use_graphs)
       if (int rc = chunk_graph<T>(c, x, b, W, n, trans, tpos, mode + 2 * (int)prec + 8 * (fused >= 0), st, Ait,
-                                  check_every, &chunk, fused))
+                                  check_every, &chunk, fused, prec))
         return rc;
     for (int replay = 1;; ++replay) {
       if (chunk)
         HIPCHECK(hipGraphLaunch(chunk, st));
       else
-        HIPCHECK((record_chunk<T>(c, x, W, n, st, Ait, check_every, fused)));
+        HIPCHECK((record_chunk<T>(c, x, W, n, st, Ait, check_every, fused, trans, prec)));
       HIPCHECK(hipMemcpyAsync(&hs, s, sizeof(TfqmrScal), hipMemcpyDeviceToHost, st));
       HIPCHECK(hipStreamSynchronize(st));
       rs.iters = base_iters + hs.iter;

@@ -102,12 +102,11 @@ struct MultiLoc {
 #define SPAN_LOOP(i, sp) \
   for (int64_t i = (sp).blk * blockDim.x + threadIdx.x; i < (sp).n2; i += (sp).nblk * blockDim.x)
 
-// The iteration's vector kernels (k_step1, k_step2, k_v) load their first
-// elements, and the partial sums they fold, before they look at the scalars,
-// and each next element before the current one is written.  On the single
-// impurity a thread has one element, so a kernel's time is its chain of loads:
-// scalars, partial sums and elements one after another took k_step2 and k_v
-// 9.0 and 8.8 us at 37,012 elements (3 us of vector traffic is not the bound).
+// k_step2 and k_v load their first elements, and the partial sums they fold,
+// before they look at the scalars.  On the single impurity a thread has one
+// element, so a kernel's time is its chain of loads: scalars, partial sums and
+// elements one after another took 9.0 and 8.8 us at 37,012 elements, together
+// 6.2 and 6.1.  (k_step1, without sums to fold, gained nothing from it.)
 template <typename V>
 __device__ inline V ld_if(const V* p, int64_t i, bool on) {
   V z;
@@ -276,42 +275,34 @@ __global__ void k_step1(const Loc loc, T* __restrict__ w, T* __restrict__ y2, co
   using V = typename W2<T>::type;
   const Span sp = loc.span();
   s += sp.q;
-  { const int64_t o = sp.off; w += o; y2 += o; v += o; aw += o; u2 += o; d += o; }
-  const int64_t step = sp.nblk * blockDim.x;
-  int64_t i = sp.blk * blockDim.x + threadIdx.x;
-  V wi, yo, a, u, b, di;
-  auto load = [&](int64_t k) {
-    const bool on = k < sp.n2;
-    wi = ld_if(reinterpret_cast<const V*>(w), k, on);
-    yo = ld_if(reinterpret_cast<const V*>(y2), k, on);
-    a = ld_if(reinterpret_cast<const V*>(aw), k, on);
-    u = ld_if(reinterpret_cast<const V*>(u2), k, on);
-    b = ld_if(reinterpret_cast<const V*>(v), k, on);
-    di = ld_if(reinterpret_cast<const V*>(d), k, on);
-  };
-  load(i);
   if (s->flag) return;
+  { const int64_t o = sp.off; w += o; y2 += o; v += o; aw += o; u2 += o; d += o; }
   const T alpha = (T)s->alpha, dcoef = (T)s->dcoef, beta = (T)s->beta;
   double ww = 0;
-  while (i < sp.n2) {
-    V y1, u1, o, wn, dn;
+  SPAN_LOOP(i, sp) {
+    V wi = reinterpret_cast<V*>(w)[i];
+    const V yo = reinterpret_cast<const V*>(y2)[i];
+    V y1;
     y1.x = wi.x + beta * yo.x;
     y1.y = wi.y + beta * yo.y;
+    const V a = reinterpret_cast<const V*>(aw)[i], u = reinterpret_cast<const V*>(u2)[i];
+    V u1;
     u1.x = a.x + beta * u.x;
     u1.y = a.y + beta * u.y;
+    const V b = reinterpret_cast<const V*>(v)[i];
+    V o;
     o.x = y1.x - alpha * b.x;
     o.y = y1.y - alpha * b.y;
-    wn.x = wi.x - alpha * u1.x;
-    wn.y = wi.y - alpha * u1.y;
+    reinterpret_cast<V*>(y2)[i] = o;
+    wi.x -= alpha * u1.x;
+    wi.y -= alpha * u1.y;
+    reinterpret_cast<V*>(w)[i] = wi;
+    const V di = reinterpret_cast<const V*>(d)[i];
+    V dn;
     dn.x = y1.x + dcoef * di.x;
     dn.y = y1.y + dcoef * di.y;
-    ww += (double)wn.x * wn.x + (double)wn.y * wn.y;
-    const int64_t at = i;
-    i += step;
-    load(i);
-    reinterpret_cast<V*>(y2)[at] = o;
-    reinterpret_cast<V*>(w)[at] = wn;
-    reinterpret_cast<V*>(d)[at] = dn;
+    reinterpret_cast<V*>(d)[i] = dn;
+    ww += (double)wi.x * wi.x + (double)wi.y * wi.y;
   }
   span_partial(ww, 0.0, partial, sp);
 }
@@ -366,12 +357,11 @@ __global__ void k_step2(const Loc loc, T* __restrict__ x, T* __restrict__ w, con
     dn.y = yi.y + dcoef * di.y;
     ww += (double)wn.x * wn.x + (double)wn.y * wn.y;
     rw += shadow(2 * i, seed) * wn.x + shadow(2 * i + 1, seed) * wn.y;
-    const int64_t at = i;
+    reinterpret_cast<V*>(x)[i] = xn;
+    reinterpret_cast<V*>(w)[i] = wn;
+    reinterpret_cast<V*>(d)[i] = dn;
     i += step;
-    load(i);
-    reinterpret_cast<V*>(x)[at] = xn;
-    reinterpret_cast<V*>(w)[at] = wn;
-    reinterpret_cast<V*>(d)[at] = dn;
+    if (i < sp.n2) load(i);
   }
   span_partial(ww, rw, partial, sp);
 }
@@ -437,14 +427,13 @@ __global__ void k_v(const Loc loc, const T* __restrict__ aw, const T* __restrict
     xn.y = xi.y + eta * di.y;
     r.x = a2.x + beta * ((T)2 * b2.x + beta * c.x);
     r.y = a2.y + beta * ((T)2 * b2.y + beta * c.y);
-    const int64_t at = i;
-    i += step;
-    load(i);
-    reinterpret_cast<V*>(x)[at] = xn;
+    reinterpret_cast<V*>(x)[i] = xn;
     if (next) {
-      reinterpret_cast<V*>(v)[at] = r;
-      sg += shadow(2 * at, seed) * r.x + shadow(2 * at + 1, seed) * r.y;
+      reinterpret_cast<V*>(v)[i] = r;
+      sg += shadow(2 * i, seed) * r.x + shadow(2 * i + 1, seed) * r.y;
     }
+    i += step;
+    if (i < sp.n2) load(i);
   }
   span_partial(sg, 0.0, partial, sp);
 }
@@ -514,7 +503,9 @@ __global__ void k_step1_fused(int64_t n2, double* __restrict__ w, double* __rest
 constexpr int kFoldThreads = 1024;
 __global__ void __launch_bounds__(kFoldThreads) k_tfq_fold(const double* __restrict__ pv, int nv,
                                                            const double* __restrict__ pa, int na, TfqmrScal* s) {
-  if (s->flag) return;
+  // the scalars and the sums are loaded together: one trip to memory, not two
+  const double s_tau = s->tau, s_alpha = s->alpha, s_rho = s->rho, s_target = s->target, s_beta = s->beta;
+  const int s_iter = s->iter, s_flag = s->flag;
   double v[6] = {0, 0, 0, 0, 0, 0};   // ||w||^2 and rt.v of step 1; ||w||^2, rt.w, rt.u2, rt.aw
   for (int t = threadIdx.x; t < nv; t += kFoldThreads) {
     v[0] += pv[2 * t];
@@ -535,6 +526,7 @@ __global__ void __launch_bounds__(kFoldThreads) k_tfq_fold(const double* __restr
 #pragma unroll
     for (int u = 0; u < 4; ++u) v[5] += l[u];
   }
+  if (s_flag) return;   // uniform
   __shared__ double red[6][kFoldThreads / 64];
 #pragma unroll
   for (int k = 0; k < 6; ++k)
@@ -551,26 +543,39 @@ __global__ void __launch_bounds__(kFoldThreads) k_tfq_fold(const double* __restr
     for (int q = 0; q < kFoldThreads / 64; ++q) v[k] += red[k][q];
   }
   const double a1 = v[0], sv = v[1], a2 = v[2], rw = v[3], ru = v[4], ra = v[5];
-  TfqmrScal t = *s;
-  half_step(&t, a1);
-  t.eta_a = t.eta;
-  t.cy = 1.0;
-  t.cd = t.dcoef;
-  half_step_rho(&t, a2, rw);
-  t.eta_b = t.flag ? 0.0 : t.eta;   // a breakdown keeps x at the first half step
-  if (t.stop) {
-    t.flag = 1;
-  } else if (!t.flag) {
-    const double sg = ra + t.beta * (2.0 * ru + t.beta * sv);
-    t.sigma = sg;
-    if (sg == 0.0) {
-      t.flag = 2;
-    } else {
-      t.alpha = t.rho / sg;
-      t.dcoef = t.theta * t.theta * t.eta / t.alpha;
-    }
+  const Half h = half_of(a1, s_tau, s_alpha);
+  // the second half step, the stop test and rho (half_step_rho on values)
+  const Half g = half_of(a2, h.tau, s_alpha);
+  const int iter = s_iter + 1;
+  const bool stop = g.tau * sqrt(2.0 * iter + 1.0) <= s_target;
+  const bool broken = !stop && s_rho == 0.0;
+  const bool on = !stop && !broken;
+  const double beta = on ? rw / s_rho : s_beta, rho = on ? rw : s_rho;
+  put_half(s, g);
+  s->iter = iter;
+  s->eta_a = h.eta;
+  s->cy = 1.0;
+  s->cd = h.dcoef;
+  s->eta_b = broken ? 0.0 : g.eta;   // a breakdown keeps x at the first half step
+  if (stop) {
+    s->stop = 1;
+    s->flag = 1;
+    return;
   }
-  *s = t;
+  if (broken) {
+    s->flag = 2;
+    return;
+  }
+  s->beta = beta;
+  s->rho = rho;
+  const double sg = ra + beta * (2.0 * ru + beta * sv);
+  s->sigma = sg;
+  if (sg == 0.0) {
+    s->flag = 2;
+    return;
+  }
+  s->alpha = rho / sg;
+  s->dcoef = g.theta * g.theta * g.eta / (rho / sg);
 }
 
 // x += eta_a d + eta_b (cy y2 + cd d): the pending update of the last fused
