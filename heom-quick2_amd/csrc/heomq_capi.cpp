@@ -341,6 +341,7 @@ struct PackedHost {
   std::vector<int32_t> lt_ados, lt_off;
   std::vector<DevEntryP> lt_ent[2];
   int lt_u = 0;
+  int lt_rec0[2] = {0, 0}, lt_recn[2] = {0, 0};   // the records the top tier's couplings use
 };
 
 constexpr int kMaxSectors = 65535;
@@ -618,10 +619,18 @@ int finish_packed_host(const Model& m, const std::vector<int64_t>& rowf, const s
       const auto& pent = w == 0 ? ph.pentf : ph.pentt;
       auto& out = ph.lt_ent[w];
       out.assign(ph.lt_ados.size() * (size_t)ph.lt_u, DevEntryP{0, -1, -1, 0, 0, 0});
-      for (size_t i = 0; i < ph.lt_ados.size(); ++i) {
-        const int64_t a = ph.lt_ados[i];
-        for (int64_t p = rows[a]; p < rows[a + 1]; ++p) out[i * ph.lt_u + (p - rows[a])] = pent[p];
-      }
+      int lo = 1 << 30, hi = -1;
+      for (const int4& blk : ph.lt_blk)
+        for (int j = 0; j < blk.y; ++j) {
+          const int64_t a = ph.lt_ados[(size_t)blk.x + j];
+          for (int64_t p = rows[a]; p < rows[a + 1]; ++p) {
+            out[(size_t)blk.x * ph.lt_u + (size_t)(p - rows[a]) * blk.y + j] = pent[p];
+            lo = std::min(lo, (int)pent[p].rec);
+            hi = std::max(hi, (int)pent[p].rec);
+          }
+        }
+      ph.lt_rec0[w] = hi < 0 ? 0 : lo;
+      ph.lt_recn[w] = hi < 0 ? 0 : hi - lo + 1;
     }
   }
   return HEOMQ_OK;
@@ -692,9 +701,10 @@ int build_packed(heomq_ctx* c, const Model& m, const std::vector<int64_t>& rowf,
     p.light_begin = ph.light_begin;
     p.light_block_ado = c->p_lblock.as<int32_t>();
     p.light_nz = c->p_lnz.as<int32_t>();
-    p.max_light_couplings = ph.max_light[w];
     p.n_lt_blocks = (int)ph.lt_blk.size();
     p.lt_u = ph.lt_u;
+    p.lt_rec0 = (uint16_t)ph.lt_rec0[w];
+    p.lt_recn = (uint16_t)ph.lt_recn[w];
     // the default form: the sector-batched top tier; below it one wave per ADO
     // where every sector is small (the single impurity: 36.8 against 89.2 us in
     // form 2 at M = 72, L = 4, 6.8 against 8.4 at L = 3), else the grouped rows
@@ -866,11 +876,12 @@ int build_spa_operator(heomq_ctx* c, const int32_t* nnz_spa, const std::vector<i
   p.light_begin = ph.light_begin;
   p.light_block_ado = so.lblock.as<int32_t>();
   p.light_nz = so.lnz.as<int32_t>();
-  p.max_light_couplings = ph.max_light[0];
   p.hg_off = so.hgoff.as<int32_t>();
   p.hg = so.hg.as<int4>();
   p.n_lt_blocks = batched ? (int)ph.lt_blk.size() : 0;
   p.lt_u = ph.lt_u;
+  p.lt_rec0 = (uint16_t)ph.lt_rec0[0];
+  p.lt_recn = (uint16_t)ph.lt_recn[0];
   p.lt_blk = batched ? so.ltblk.as<int4>() : nullptr;
   p.lt_off = batched ? so.ltoff.as<int32_t>() : nullptr;
   p.lt_id = batched ? so.ltados.as<int32_t>() : nullptr;
@@ -1002,11 +1013,12 @@ int build_trun(heomq_ctx* c) {
   p.light_begin = ph.light_begin;
   p.light_block_ado = tr.lblock.as<int32_t>();
   p.light_nz = tr.lnz.as<int32_t>();
-  p.max_light_couplings = ph.max_light[0];
   p.hg_off = tr.hgoff.as<int32_t>();
   p.hg = tr.hg.as<int4>();
   p.n_lt_blocks = batched ? (int)ph.lt_blk.size() : 0;
   p.lt_u = ph.lt_u;
+  p.lt_rec0 = (uint16_t)ph.lt_rec0[0];
+  p.lt_recn = (uint16_t)ph.lt_recn[0];
   p.lt_blk = batched ? tr.ltblk.as<int4>() : nullptr;
   p.lt_off = batched ? tr.ltoff.as<int32_t>() : nullptr;
   p.lt_id = batched ? tr.ltados.as<int32_t>() : nullptr;

@@ -113,7 +113,6 @@ struct DevPacked {
   const int32_t* light_block_ado = nullptr;  // per light block: index into light_nz of the ADO holding its
                                              // first element (+ one entry for the end); a block spans at most
                                              // 257 of these ADOs
-  int max_light_couplings = 0;       // largest coupling count of a top-tier ADO (<= 8)
   // Grouped form of the ADOs below the top tier (the reference's
   // accumulate-then-apply order, calc_ax_tfqmr_omp.f90:289-353): the row of
   // heavy ADO a is sorted so that entries sharing a gather map (one c
@@ -127,9 +126,10 @@ struct DevPacked {
   // Sector-batched top tier: light block b takes the top-tier ADOs i =
   // lt_blk[b].x .. + lt_blk[b].y - 1 of a list sorted by sector, all of
   // sector lt_blk[b].w with lt_blk[b].z elements each; lt_off[i] is ADO i's
-  // first packed element, lt_id[i] the ADO, lt_ent[i * lt_u + r] its
-  // coupling r (map -1 past its last), lt_u the most couplings of a top-tier
-  // ADO.  Null: the top tier runs in packed-element order (light_block_ado).
+  // first packed element, lt_id[i] the ADO, lt_ent[lt_blk[b].x * lt_u +
+  // r * lt_blk[b].y + j] coupling r of the block's ADO j (map -1 past its last;
+  // neighbouring lanes read neighbouring entries), lt_u the most couplings of
+  // a top-tier ADO, [lt_rec0, lt_rec0 + lt_recn) the records they use.  Null: the top tier runs in packed-element order (light_block_ado).
   const int4* lt_blk = nullptr;
   const int32_t* lt_off = nullptr;
   const int32_t* lt_id = nullptr;
@@ -148,6 +148,7 @@ struct DevPacked {
   const int16_t* hq = nullptr;
   const double* hc = nullptr;        // complex coefficients of i(HX - XH)
   const int2* maps = nullptr;        // paired gather maps {left, right}
+  uint16_t lt_rec0 = 0, lt_recn = 0;
   int wide = 0;                      // 1: more than kNarrowElems elements, gathered at 64-bit addresses
   // batch of problems sharing every structural table (grid y = problem):
   // problem p's vectors start p * vstride complex elements in, its records,

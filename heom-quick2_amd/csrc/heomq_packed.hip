@@ -830,15 +830,22 @@ __device__ inline void heavy_wave(const DevPacked& op, const Coefs cf_p, const T
 // the entries' signs on the coefficients, and the lanes read them there: 12
 // global loads per lane instead of 25 at d = 16, where the loads' address
 // path, not their bytes, was the bound.  With few lanes per ADO (d = 4) each
-// lane loads its own.  The lane's own element of x goes through LDS, where the
+// lane loads its own entries, and the coefficients come from LDS, where the
+// block stages the top tier's records (M of them forward, up to 3 M
+// transposed): two 16-byte loads per coupling of a lane less (FEW: the kernels
+// of the wave form, whose sectors are all small; FP32 at M = 64, L = 4: 25.4 ->
+// 23.8 us.  In the other forms' kernels the same path cost 3 %, 34.2 -> 35.3 us
+// at two impurities, M = 96, and they gather before the barrier).  The lane's own element of x goes through LDS, where the
 // sector's commutator rows (staged once per block) read their neighbours.
 constexpr int kLStage = 128;   // couplings of one block staged in LDS
 constexpr int kLightU = 3;     // of one lane in flight
 constexpr size_t kLOffHc = 0, kLOffX = kLOffHc + 256 * 16, kLOffL = kLOffX + 256 * 16,
                  kLOffR = kLOffL + kLStage * 16, kLOffBm = kLOffR + kLStage * 16, kLOffG = kLOffBm + kLStage * 8,
                  kLSmem = kLOffG + kLStage * 16;
+// records whose coefficients a block of few lanes per ADO stages instead
+constexpr int kLRecs = kLStage * (16 + 16 + 8 + 16) / 32;
 
-template <typename T, bool TRANS, bool WIDE, bool STAGE = false, class Ep = NoEpi>
+template <typename T, bool TRANS, bool WIDE, bool STAGE = false, class Ep = NoEpi, bool FEW = false>
 __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const T* __restrict__ x,
                                     T* __restrict__ y, int64_t zero_at, int bid, char* smem, bool scaled,
                                     StageOut* so = nullptr, Ep* ep = nullptr) {
@@ -855,6 +862,8 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
   const int dd = op.d * op.d;
   const int W = op.hell_w;
   const bool stg = cnt * U <= kLStage;        // block-uniform
+  const bool ldsc = FEW && !stg && op.lt_recn > 0 && op.lt_recn <= kLRecs;
+  double2* s_cf = reinterpret_cast<double2*>(smem + kLOffL);   // over the staged couplings' place
   const bool hst = W > 0 && nnz * W <= 256;   // the sector's commutator rows fit the LDS table
   const int j = div_by(threadIdx.x, div_inv(nnz)), t = threadIdx.x - j * nnz;   // 1 <= nnz <= 256 (host check)
   const bool act = j < cnt;
@@ -864,15 +873,36 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
   DevEntryP e0{0, -1, -1, 0, 0, 0};
   int ida = 0;
   if (stg) {
-    if (threadIdx.x < cnt * U) e0 = op.lt_ent[(int64_t)bd.x * U + threadIdx.x];
+    if (threadIdx.x < cnt * U) e0 = op.lt_ent[(int64_t)bd.x * U + threadIdx.x];   // coupling tid / cnt of ADO tid % cnt
     if (threadIdx.x < cnt) ida = op.lt_id[bd.x + threadIdx.x];
   }
+  // the lane's own couplings, two at a time: entries, then map values and
+  // coefficients, then the four elements, then the sums
+  auto direct = [&]() {
+    const DevEntryP* en = op.lt_ent + (int64_t)bd.x * U + j;
+    for (int r0 = 0; r0 < U; r0 += 2) {
+      DevEntryP e[2];
+      CoefLR cf[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) e[q] = r0 + q < U ? en[(r0 + q) * cnt] : DevEntryP{0, -1, -1, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if (e[q].map < 0) cf[q] = CoefLR{};
+        else if (ldsc) cf[q] = CoefLR{s_cf[2 * (e[q].rec - op.lt_rec0)], s_cf[2 * (e[q].rec - op.lt_rec0) + 1]};
+        else cf[q] = load_coef(cf_p.rec, e[q].rec);
+      }
+      coupling_block<T, TRANS, WIDE, 2>(e, cf, 2, op.maps, xs, t, zero_at, ar, ai);
+    }
+  };
   if (act) base = op.lt_off[i];
   if (hst && threadIdx.x < nnz * W)   // rows of one sector are consecutive
     s_hc[threadIdx.x] = reinterpret_cast<const double2*>(cf_p.hc_ell)[(int64_t)s * dd * W + threadIdx.x];
   if (act) s_x[threadIdx.x] = ld<T, TRANS>(xv, (int64_t)base + t, zero_at);
   if (stg) {
-    if (threadIdx.x < cnt * U) st.put(threadIdx.x, e0, cf_p.rec);
+    if (threadIdx.x < cnt * U) {   // an ADO's couplings side by side, for constant offsets below
+      const int r = div_by(threadIdx.x, div_inv(cnt));
+      st.put((threadIdx.x - r * cnt) * U + r, e0, cf_p.rec);
+    }
     if (threadIdx.x < cnt) {
       const double2 g = reinterpret_cast<const double2*>(cf_p.gam)[ida];
       V gv;
@@ -880,22 +910,16 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
       gv.y = (T)g.y;
       s_g[threadIdx.x] = gv;
     }
-  } else if (act) {
-    const int64_t a = op.lt_id[i];
-    gr = (T)cf_p.gam[2 * a];
-    gi = (T)cf_p.gam[2 * a + 1];
-    // the lower-tier couplings, two at a time: entries, then map values and
-    // records, then the four elements, then the sums
-    const DevEntryP* en = op.lt_ent + i * U;
-    for (int r0 = 0; r0 < U; r0 += 2) {
-      DevEntryP e[2];
-      CoefLR cf[2];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) e[q] = r0 + q < U ? en[r0 + q] : DevEntryP{0, -1, -1, 0, 0, 0};
-#pragma unroll
-      for (int q = 0; q < 2; ++q) cf[q] = e[q].map >= 0 ? load_coef(cf_p.rec, e[q].rec) : CoefLR{};
-      coupling_block<T, TRANS, WIDE, 2>(e, cf, 2, op.maps, xs, t, zero_at, ar, ai);
+  } else {
+    if (act) {
+      const int64_t a = op.lt_id[i];
+      gr = (T)cf_p.gam[2 * a];
+      gi = (T)cf_p.gam[2 * a + 1];
     }
+    if (ldsc)
+      for (int k = threadIdx.x; k < 2 * op.lt_recn; k += 256)
+        s_cf[k] = reinterpret_cast<const double2*>(cf_p.rec + op.lt_rec0 + (k >> 1))[k & 1];
+    if (!FEW && act) direct();
   }
   __syncthreads();
   if (!act) return;   // after the only barrier
@@ -904,6 +928,8 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
     gi = s_g[j].y;
     for (int r0 = 0; r0 < U; r0 += kLightU)
       staged_block<T, TRANS, WIDE, kLightU>(st, j * U + r0, U - r0, op.maps, xs, t, zero_at, ar, ai);
+  } else if (FEW) {
+    direct();
   }
   T csr = 0, csi = 0;
   const V* xw = s_x + j * nnz;   // this ADO's elements
@@ -1001,7 +1027,7 @@ __device__ inline void apply_block(const DevPacked& op, int64_t p, int64_t bx, c
     else
       heavy_body<T, TRANS, WIDE, false, Ep>(op, cf, x, y, zero_at, rdo, a, smem, scaled, nullptr, ep);
   } else if (sector) {
-    light_sector<T, TRANS, WIDE, false, Ep>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, nullptr, ep);
+    light_sector<T, TRANS, WIDE, false, Ep, (FORM >= 0 && (FORM & 4) != 0)>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, nullptr, ep);
   } else {
     light_body<T, TRANS, WIDE, Ep>(op, cf, x, y, zero_at, (int)(bx - hb), smem, scaled, ep);
   }
