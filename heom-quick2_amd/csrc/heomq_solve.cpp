@@ -1089,16 +1089,12 @@ int rk4_steps(double* x, int64_t n, double* rho0, double* tmp, double* k, double
   const double dt2 = dt / 2, dt3 = dt / 3, dt6 = dt / 6;
   for (int step = 0; step < nstep; ++step) {
     const double t = t0 + step * dt;
-    HIPCHECK(hipMemcpyAsync(rho0, x, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-    if (int rc = deriv(t, rho0, k)) return rc;
-    HIPCHECK(vec_lincomb3(st, n, tmp, 1.0, rho0, dt2, k, 0.0, nullptr));
-    HIPCHECK(vec_lincomb3(st, n, x, 1.0, x, dt6, k, 0.0, nullptr));
+    if (int rc = deriv(t, x, k)) return rc;
+    HIPCHECK(rk4_stage(st, n, true, x, rho0, tmp, k, dt2, dt6));
     if (int rc = deriv(t + dt2, tmp, k)) return rc;
-    HIPCHECK(vec_lincomb3(st, n, tmp, 1.0, rho0, dt2, k, 0.0, nullptr));
-    HIPCHECK(vec_lincomb3(st, n, x, 1.0, x, dt3, k, 0.0, nullptr));
+    HIPCHECK(rk4_stage(st, n, false, x, rho0, tmp, k, dt2, dt3));
     if (int rc = deriv(t + dt2, tmp, k)) return rc;
-    HIPCHECK(vec_lincomb3(st, n, tmp, 1.0, rho0, dt, k, 0.0, nullptr));
-    HIPCHECK(vec_lincomb3(st, n, x, 1.0, x, dt3, k, 0.0, nullptr));
+    HIPCHECK(rk4_stage(st, n, false, x, rho0, tmp, k, dt, dt3));
     if (int rc = deriv(t + dt, tmp, k)) return rc;
     HIPCHECK(vec_lincomb3(st, n, x, 1.0, x, dt6, k, 0.0, nullptr));
   }
@@ -1163,9 +1159,15 @@ int cheby_steps(double* x, int64_t n, double* pm2, double* pm1, double* lp, cons
 
 int rk4_packed_core(heomq_ctx* c, double* xp, double t0, double dt, int nstep, hipStream_t st,
                     const std::vector<double*>& v) {
+  // two of a step's four derivatives (and often the next step's first) share a
+  // time: the field's rates are formed once per time
+  DevPacked op;
+  double at = std::numeric_limits<double>::quiet_NaN();
   auto deriv = [&](double t, const double* in, double* out) -> int {
-    DevPacked op;
-    if (int rc = packed_prop_op(c, t, st, op)) return rc;
+    if (!(t == at)) {
+      if (int rc = packed_prop_op(c, t, st, op)) return rc;
+      at = t;
+    }
     HIPCHECK(launch_apply_packed_f64(op, in, out, false, st));
     return HEOMQ_OK;
   };
@@ -1212,9 +1214,13 @@ int heomq_rk4_at(heomq_ctx* c, double* x, double t0, double dt, int nstep, void*
   }
   const int64_t n = 2 * c->N * c->d * c->d;
   if (int rc = carve<double>(c->ws64, n, 3, v)) return rc;
+  DevOperator op;
+  double at = std::numeric_limits<double>::quiet_NaN();
   auto deriv = [&](double t, const double* in, double* out) -> int {
-    DevOperator op;
-    if (int rc = operator_at(c, t, st, op)) return rc;
+    if (!(t == at)) {
+      if (int rc = operator_at(c, t, st, op)) return rc;
+      at = t;
+    }
     HIPCHECK(launch_apply_f64(op, in, out, -1, st));
     return HEOMQ_OK;
   };

@@ -6,6 +6,7 @@
 // A whole iteration is launch-only (no host round trip) and deterministic.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "heomq_shadow.hpp"
@@ -723,6 +724,26 @@ __global__ void k_lincomb3(int64_t n, double* __restrict__ out, double a, const 
   }
 }
 
+// An RK4 stage's two vector updates in one pass, the derivative k read once:
+// tmp = rho0 + a k (the next stage's input), x += b k; the first stage takes
+// rho0 = x and stores it.  7 launches and a copy per step become 4.
+__global__ void k_rk4_stage(int64_t n2, int first, double2* __restrict__ x, double2* __restrict__ rho0,
+                            double2* __restrict__ tmp, const double2* __restrict__ k, double a, double b) {
+  GRID_LOOP(i, n2) {
+    const double2 xi = x[i], ki = k[i];
+    double2 r = xi;
+    if (first) rho0[i] = xi;
+    else r = rho0[i];
+    r.x += a * ki.x;
+    r.y += a * ki.y;
+    tmp[i] = r;
+    double2 o = xi;
+    o.x += b * ki.x;
+    o.y += b * ki.y;
+    x[i] = o;
+  }
+}
+
 // Projection onto the physical sector: zero the elements a tier-n ADO cannot
 // hold (parity(i) + parity(j) + n odd) and Hermitianise the tier-0 block.
 template <typename T>
@@ -955,6 +976,17 @@ hipError_t vec_set_pattern(hipStream_t st, double* v, int64_t stride, int nprob,
 }
 hipError_t vec_set_elem(hipStream_t st, double* v, int64_t off, double val) {
   hipLaunchKernelGGL((k_set_elem<double>), dim3(1), dim3(64), 0, st, v, off, val);
+  return hipGetLastError();
+}
+
+hipError_t rk4_stage(hipStream_t st, int64_t n, bool first, double* x, double* rho0, double* tmp, const double* k,
+                     double a, double b) {
+  const int64_t n2 = n / 2;
+  if (n2 <= 0) return hipSuccess;
+  const unsigned grid = (unsigned)std::min<int64_t>((n2 + 255) / 256, 4096);
+  hipLaunchKernelGGL(k_rk4_stage, dim3(grid), dim3(256), 0, st, n2, first ? 1 : 0, reinterpret_cast<double2*>(x),
+                     reinterpret_cast<double2*>(rho0), reinterpret_cast<double2*>(tmp),
+                     reinterpret_cast<const double2*>(k), a, b);
   return hipGetLastError();
 }
 

@@ -169,6 +169,9 @@ struct SetPattern {
   double val[64];
 };
 hipError_t vec_set_pattern(hipStream_t, double* v, int64_t stride, int nprob, const SetPattern& pat);
+// tmp = rho0 + a k, x += b k on vectors of n reals (complex, n even); first: rho0 = x is stored too
+hipError_t rk4_stage(hipStream_t, int64_t n, bool first, double* x, double* rho0, double* tmp, const double* k,
+                     double a, double b);
 hipError_t vec_lincomb3(hipStream_t, int64_t n, double* out, double a, const double* x, double b,
                         const double* y, double c, const double* z);
 
