@@ -369,10 +369,9 @@ __device__ inline void staged_block(const StagedLds<T>& st, int k, int nv, const
 // Top-tier ADOs: one thread per packed element.  A block stages in LDS the
 // headers (offset, first and last entry, sector, gamma) of the non-empty ADOs
 // it covers (at most 257, checked when the tables are built) and its own 256
-// elements of x (the commutator's neighbours); the couplings are then read U
-// at a time (U = min(the top tier's coupling count, 2): two couplings in
-// flight keep the kernel at 72 VGPRs, 7 waves per SIMD; the coefficient
-// records come from L2, which holds them for every block).
+// elements of x (the commutator's neighbours); the couplings are then read
+// two at a time (two in flight keep the kernel at 72 VGPRs, 7 waves per SIMD;
+// the coefficient records come from L2, which holds them for every block).
 // LDS carve-up of the light and heavy bodies (they share one buffer).
 constexpr size_t kAlign16(size_t b) { return (b + 15) / 16 * 16; }
 constexpr size_t kLightOffP0 = kAlign16(257 * 8), kLightOffP1 = kLightOffP0 + kAlign16(257 * 8),
@@ -992,6 +991,13 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
 // the top tier's elements, so the two phases overlap on the device.  The LDS
 // buffer allows 7 blocks per CU; the register budget is held to the same 7
 // waves per SIMD (72 VGPRs).
+//
+// Bound by no one unit: at two-impurity size (M = 112, L = 3, 1.8 M elements)
+// the address units are busy 57 % of the time, the vector units 45 %, and the
+// Infinity Cache delivers 166 MB (the top tier four times); each workgroup is
+// a chain of five or six dependent loads.  FP64 forward 58.7 us (form 2, the
+// former default) -> 50.5 us (form 3), transposed 64.6 -> 52.3; single impurity
+// M = 72, L = 4: 83.4 us (form 2) -> 34.7 us (form 6).
 constexpr size_t kApplySmem1 = kGSmem > kLSmem ? kGSmem : kLSmem;
 constexpr size_t kApplySmem = kApplySmem0 > kApplySmem1 ? kApplySmem0 : kApplySmem1;
 
@@ -1564,7 +1570,10 @@ __device__ inline void tfq_partials(double r0, double r1, double r2, const TfqEp
 
 // The plain (or Jacobi-scaled) apply with a TFQMR iteration's vector work on
 // its outputs (TfqPut): k_step2 and the v update of k_v and their launches are
-// gone from the iteration, as in the preconditioned one below.
+// gone from the iteration, as in the preconditioned one below (single impurity,
+// 37,012 elements: 35.4 -> 27.1 us of kernels per iteration; 8.0 and 7.3 us for
+// the two applies with their epilogues against 7.2 without).  6 waves per SIMD:
+// 72 VGPRs spilled 44 bytes per lane.
 template <bool TRANS, int FORM, int KIND>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 k_apply_packed_tfq(const DevPacked op, const double* __restrict__ x, double* __restrict__ y, int64_t zero_at, int rdo,

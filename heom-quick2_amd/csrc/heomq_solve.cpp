@@ -958,7 +958,7 @@ int heomq_apply_packed_precond(heomq_ctx* c, const double* xp, double* yp, int t
   jc.ejac = c->prec_shift;
   if (form == 4) {
     if (c->trun.built || !apply_jac_fusable(op, jc))
-      return fail(HEOMQ_UNSUPPORTED, "the fused preconditioned apply needs apply form 2 or 6 without the wave form "
+      return fail(HEOMQ_UNSUPPORTED, "the fused preconditioned apply needs a sector-batched apply form without the wave form "
                                      "and the ADO-aligned inverse");
     HIPCHECK(launch_apply_packed_jac(op, jc, xp, yp, rdo, st));
     return HEOMQ_OK;

@@ -459,9 +459,10 @@ class Context:
         return C.c_void_p(v.data_ptr())
 
     def set_precond(self, mode: int, shift: float | None = None):
-        """Left preconditioning of forward steady solves: -1 automatic (Jacobi
-        scaling for diagonal H, block Jacobi otherwise), 0 none, 1 Jacobi
-        scaling, 2 block Jacobi with the given shift (None / 0: default)."""
+        """Left preconditioning of steady solves: -1 automatic (Jacobi scaling
+        for diagonal H, block Jacobi otherwise), 0 none, 1 Jacobi scaling, 2
+        block Jacobi with the given shift (None / 0: default).  Transposed
+        solves take the Jacobi scaling only."""
         check(lib().heomq_ctx_set_precond(self._h, int(mode)))
         if shift is not None:
             check(lib().heomq_ctx_set_precond_shift(self._h, float(shift)))
@@ -477,7 +478,9 @@ class Context:
 
     def set_precond_fusion(self, enable: bool):
         """Block-Jacobi-preconditioned applies as one fused launch where the
-        apply form allows it (default on; the same bits as the two kernels)."""
+        apply form allows it (the same bits as the two kernels), and solver
+        iterations with their vector work in the operator launches (default
+        on)."""
         check(lib().heomq_ctx_set_precond_fusion(self._h, int(enable)))
 
     def set_trun_der(self, enable: bool = True):
@@ -763,8 +766,8 @@ class Context:
                      raise_on_fail=True):
         """TFQMR steady state on the device; returns (x, stats dict): iters,
         applies, relres, seconds, status, precond (the left preconditioner
-        the iteration ended with) and fused_iteration (block-Jacobi
-        iterations ran with their vector work in the operator launches)."""
+        the iteration ended with) and fused_iteration (iterations ran with
+        their vector work in the operator launches)."""
         t = self.torch
         x = self.initial_guess() if x is None else x
         stats = np.zeros(_lib.STATS_LEN)

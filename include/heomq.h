@@ -191,15 +191,16 @@ int heomq_ctx_set_presmooth(heomq_ctx* c, int enable);
 /* Block-Jacobi-preconditioned packed applies (the steady solve's iteration,
  * heomq_apply_packed_precond) run as one fused launch, the inverse applied to
  * each workgroup's ADOs before anything is written, when the forward apply
- * form has the sector-batched top tier and sliced heavy rows (enable = 1, the
- * default; the results are the same bits); 0 always runs the apply, then the
- * inverse.  The same switch fuses each Chebyshev term of the packed
+ * form has the sector-batched top tier and a workgroup per heavy row (enable =
+ * 1, the default; the same values); 0 always runs the apply, then the
+ * inverse.  The same switch lets the plain and Jacobi-scaled solver iterations
+ * carry their vector work in the apply, and fuses each Chebyshev term of the packed
  * propagators (the apply's output folded into the recurrence and the sum,
  * one launch, the same bits).  No counterpart in the reference. */
 int heomq_ctx_set_precond_fusion(heomq_ctx* c, int enable);
-/* Left preconditioning of the forward steady-state TFQMR on the packed
- * layout: 0 none; 1 Jacobi (diagonal) scaling, default right-hand side only;
- * 2 block Jacobi, (shift - S_K)^-1 per ADO with S_K the same-tier operator
+/* Left preconditioning of the steady-state TFQMR on the packed layout: 0 none;
+ * 1 Jacobi (diagonal) scaling, any right-hand side, forward and transposed; 2
+ * block Jacobi (forward solves; transposed ones run unpreconditioned), (shift - S_K)^-1 per ADO with S_K the same-tier operator
  * (the sweep operator of jacobi/calc_ax_jacobi_omp.f90 used as M^-1); -1
  * automatic: 1 when H is diagonal in the occupation basis (the single-
  * impurity model), 2 otherwise.  The convergence test always uses the
@@ -274,8 +275,8 @@ int heomq_apply_packed_raw_f32(heomq_ctx* c, const float* xp, float* yp, int tra
  * apply, then the two-kernel transform; 3: apply, then the LDS-window kernel
  * (when every ADO range a 256-element block touches fits its LDS); 4: one
  * fused launch, the inverse applied in each apply workgroup to its whole
- * ADOs (apply forms 2 and 6 without the wave form, d <= 16, the ADO-aligned
- * inverse; the same bits as form 1), HEOMQ_UNSUPPORTED otherwise.  All forms
+ * ADOs (the sector-batched apply forms without the wave form, d <= 16, the
+ * ADO-aligned inverse), HEOMQ_UNSUPPORTED otherwise.  All forms
  * compute the same values.  No counterpart in the reference. */
 int heomq_apply_packed_precond(heomq_ctx* c, const double* xp, double* yp, int trace, int form, void* stream);
 /* The same operator as heomq_apply_packed_precond form 1, with no allocation:
@@ -323,10 +324,10 @@ int heomq_calcderiv(heomq_ctx* c, const double* rhotmp_host, double* rhorhs_host
  * stats (HEOMQ_STATS_LEN): [0] iterations, [1] applies, [2] final relative
  * residual, [3] seconds, [4] the left preconditioner the iteration ended
  * with (0 none, 1 Jacobi scaling, 2 block Jacobi), [5] length of the real
- * vector iterated on, [6] 1 when block-Jacobi iterations ran with their
- * vector work carried by the fused preconditioned launches (FP64 forward
- * solve, fusable apply form, fusion on: heomq_ctx_set_precond_fusion; the
- * same iterates in exact arithmetic, reductions in another order), [7] 0.
+ * vector iterated on, [6] 1 when iterations ran with their vector work
+ * carried by the operator launches (FP64 packed solve; with block Jacobi a
+ * fusable apply form; fusion on: heomq_ctx_set_precond_fusion; the same
+ * iterates in exact arithmetic, reductions in another order), [7] 0.
  * Returns HEOMQ_NOT_CONVERGED if maxiter hit.
  * ------------------------------------------------------------------------- */
 int heomq_solve_steady(heomq_ctx* c, double* x, const double* b, double tol,
