@@ -708,11 +708,12 @@ int build_packed(heomq_ctx* c, const Model& m, const std::vector<int64_t>& rowf,
     // the default form: the sector-batched top tier; below it one wave per ADO
     // where every sector is small (the single impurity: 36.8 against 89.2 us in
     // form 2 at M = 72, L = 4, 6.8 against 8.4 at L = 3), else the grouped rows
-    // (two impurities, M = 112, L = 3: 50.5 against 56.2 us, 14.5 against 16.5
-    // at M = 64).  The autotuner (heomq_ctx_autotune) picks per operator,
+    // forward (two impurities, M = 112, L = 3: 50.5 against 56.2 us, 14.5 against
+    // 16.5 at M = 64) and the sliced ones transposed (52 against 53 us, 7.5
+    // against 8.1 at L = 2, 15.9 against 15.4 at M = 64).  The autotuner (heomq_ctx_autotune) picks per operator,
     // HEOMQ_APPLY_FORM forces one.
     const char* form = std::getenv("HEOMQ_APPLY_FORM");
-    set_apply_form(c, w, form ? std::atoi(form) : (c->heavy_wave_ok ? 6 : 3));
+    set_apply_form(c, w, form ? std::atoi(form) : (c->heavy_wave_ok ? 6 : (w == 0 ? 3 : 2)));
   }
   return HEOMQ_OK;
 }
