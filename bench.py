@@ -194,7 +194,7 @@ def main():
     achieved = bytes_alg / t_apply / 1e9
     plain = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
              "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic(args.workload),
-             "kernel": "k_apply_packed<double,false,2>", "t_apply_us": round(t_apply * 1e6, 2),
+             "kernel": "k_apply_packed<double, false>", "t_apply_us": round(t_apply * 1e6, 2),
              "form": tuned["forward"], "autotune_us": tuned["times_us"],
              "bytes_alg": bytes_alg, "packed_elems": P, "dense_elems": info["dense"],
              "dense_equiv_GBs": round(dense_bytes / t_apply / 1e9, 1)}
@@ -209,7 +209,7 @@ def main():
             roofline = {"bound": "hbm", "achieved": round(a_f, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(a_f / HBM_PEAK_GBS, 4),
                         "traffic": measured_traffic(args.workload, "precond_apply"),
-                        "kernel": "k_apply_packed_jac<true, 0> (packed apply + block-Jacobi inverse, one launch)",
+                        "kernel": "k_apply_packed_jac<true, 0, false> (packed apply + block-Jacobi inverse, one launch)",
                         "t_apply_us": round(t_fused * 1e6, 2), "form": tuned["forward"], "bytes_alg": bytes_alg,
                         "packed_elems": P, "plain_apply": plain}
 
