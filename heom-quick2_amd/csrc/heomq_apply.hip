@@ -145,13 +145,6 @@ struct DenseLds {
   }
 };
 
-template <typename T>
-__device__ inline int tier_parity(const DevOperator& op, int64_t a) {
-  int n = 0;
-  while (n + 1 < op.tb.ntier && op.tb.first[n + 1] <= a) ++n;
-  return n & 1;
-}
-
 // Blocks [0, n_heavy) take one ADO below the top tier each; the rest take
 // `run` groups of 256 / min(d*d, 256) consecutive top-tier ADOs.
 //
@@ -169,8 +162,7 @@ __device__ inline int tier_parity(const DevOperator& op, int64_t a) {
 // built per context: not kept.
 template <int D, typename T, bool TRANS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 16 ? 6 : 2)))
-k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_t trace_pos, int project,
-        int64_t n_heavy, int run, int light_max) {
+k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_t trace_pos, int run) {
   using V = typename V2<T>::type;
   constexpr int E = D * D;
   constexpr int LANES = E < 256 ? E : 256;
@@ -184,6 +176,8 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
   const int slot = APB > 1 ? tid / LANES : 0, lane = tid - slot * LANES;   // one ADO per group: uniform addresses
   const V* __restrict__ xv = reinterpret_cast<const V*>(x);
   V* __restrict__ yv = reinterpret_cast<V*>(y);
+  const int64_t n_heavy = op.n_heavy;
+  const int light_max = op.light_max;
   tab.stage(op);
 
   if ((int64_t)blockIdx.x < n_heavy) {   // block-uniform
@@ -195,7 +189,6 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
     }
     const T gr = (T)op.gam[2 * a], gi = (T)op.gam[2 * a + 1];
     const int64_t p0 = op.rowptr[a], p1 = op.rowptr[a + 1];
-    const int tpar = project ? tier_parity<T>(op, a) : 0;
     for (int k = 0; k < EPT; ++k) {
       const int e = lane + k * LANES;
       T ar = 0, ai = 0;
@@ -228,9 +221,7 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
         ai = xs[tid].y;
       }
       if (slot == 0) {
-        V o{ar, ai};
-        if (project && ((op.parity[e % D] + op.parity[e / D] + tpar) & 1)) o = V{0, 0};
-        yv[a * E + e] = o;
+        yv[a * E + e] = V{ar, ai};
       }
     }
     return;
@@ -263,7 +254,6 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
   for (int r = 0; r < nr; ++r) {
     const int64_t a = a0 + (int64_t)r * APB + slot;
     const bool active = a < op.n_ado;
-    const int tpar = project ? tier_parity<T>(op, a) : 0;
     V* xr = EPT == 1 ? &xs[(r & 1) * 256] : xs;
     if (EPT == 1) {
       xr[tid] = TRANS && a == trace_pos && lane == op.trace_elem ? V{0, 0} : own;
@@ -292,27 +282,9 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
       if (k == 0) __syncthreads();   // xs is staged
       if (active) {
         tab.template same_tier<T>(op, xr + slot * E, g.x, g.y, e % D, e / D, ar, ai);
-        V o{ar, ai};
-        if (project && ((op.parity[e % D] + op.parity[e / D] + tpar) & 1)) o = V{0, 0};
-        yv[a * E + e] = o;
+        yv[a * E + e] = V{ar, ai};
       }
     }
-  }
-}
-
-// y0 = (y0 + y0^H) / 2 on the tier-0 block (one workgroup).
-template <typename T>
-__global__ void k_hermitize_block0(T* __restrict__ y, int d) {
-  for (int e = threadIdx.x; e < d * d; e += blockDim.x) {
-    const int i = e % d, j = e / d;
-    if (i > j) continue;
-    const int t = j + i * d;
-    const T re = (T)0.5 * (y[2 * e] + y[2 * t]);
-    const T im = (T)0.5 * (y[2 * e + 1] - y[2 * t + 1]);
-    y[2 * e] = re;
-    y[2 * e + 1] = im;
-    y[2 * t] = re;
-    y[2 * t + 1] = -im;
   }
 }
 
@@ -346,25 +318,19 @@ __global__ void k_trace_trn(const T* __restrict__ w, T* __restrict__ z, int d, i
 constexpr int kLightRunMax = 8, kLightBlocksMin = 4096;
 
 template <int D, typename T>
-static hipError_t launch_d(const DevOperator& op, const T* x, T* y, int64_t trace_pos, hipStream_t s,
-                           bool project) {
+static hipError_t launch_d(const DevOperator& op, const T* x, T* y, int64_t trace_pos, hipStream_t s) {
   constexpr int E = D * D;
   constexpr int LANES = E < 256 ? E : 256;
   constexpr int APB = 256 / LANES;
   if (op.n_ado <= 0) return hipSuccess;
-  // heavy: every tier below the top one (the only tier of a tier-0 hierarchy)
-  const int64_t n_heavy = op.tb.ntier >= 2 ? op.tb.first[op.tb.ntier - 1] : op.n_ado;
-  const int64_t groups = (op.n_ado - n_heavy + APB - 1) / APB;
+  const int64_t groups = (op.n_ado - op.n_heavy + APB - 1) / APB;
   const int64_t fit = std::max<int64_t>(1, kStage / (APB * (int64_t)op.light_max));   // runs whose couplings fit the stage
   const int run = (int)std::min({fit, (int64_t)kLightRunMax, std::max<int64_t>(1, groups / kLightBlocksMin)});
-  const int64_t blocks = n_heavy + (groups + run - 1) / run;
-  const int pj = project ? 1 : 0;
+  const int64_t blocks = op.n_heavy + (groups + run - 1) / run;
   if (op.transposed)
-    hipLaunchKernelGGL((k_apply<D, T, true>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, pj,
-                       n_heavy, run, op.light_max);
+    hipLaunchKernelGGL((k_apply<D, T, true>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, run);
   else
-    hipLaunchKernelGGL((k_apply<D, T, false>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, pj,
-                       n_heavy, run, op.light_max);
+    hipLaunchKernelGGL((k_apply<D, T, false>), dim3((unsigned)blocks), dim3(256), 0, s, op, x, y, trace_pos, run);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   if (trace_pos >= 0) {
@@ -373,34 +339,25 @@ static hipError_t launch_d(const DevOperator& op, const T* x, T* y, int64_t trac
     else
       hipLaunchKernelGGL((k_trace_fwd<T>), dim3(1), dim3(64), 0, s, x, y, D, trace_pos, op.trace_elem);
     err = hipGetLastError();
-    if (err != hipSuccess) return err;
-  }
-  if (project) {
-    hipLaunchKernelGGL((k_hermitize_block0<T>), dim3(1), dim3(256), 0, s, y, D);
-    err = hipGetLastError();
   }
   return err;
 }
 
 template <typename T>
-static hipError_t launch_any(const DevOperator& op, const T* x, T* y, int64_t trace_pos, hipStream_t s,
-                             bool project) {
-  if (project && !op.parity) return hipErrorInvalidValue;
+static hipError_t launch_any(const DevOperator& op, const T* x, T* y, int64_t trace_pos, hipStream_t s) {
   switch (op.d) {
-    case 4: return launch_d<4, T>(op, x, y, trace_pos, s, project);
-    case 16: return launch_d<16, T>(op, x, y, trace_pos, s, project);
-    case 64: return launch_d<64, T>(op, x, y, trace_pos, s, project);
+    case 4: return launch_d<4, T>(op, x, y, trace_pos, s);
+    case 16: return launch_d<16, T>(op, x, y, trace_pos, s);
+    case 64: return launch_d<64, T>(op, x, y, trace_pos, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-hipError_t launch_apply_f64(const DevOperator& op, const double* x, double* y, int64_t trace_pos, hipStream_t s,
-                            bool project) {
-  return launch_any<double>(op, x, y, trace_pos, s, project);
+hipError_t launch_apply_f64(const DevOperator& op, const double* x, double* y, int64_t trace_pos, hipStream_t s) {
+  return launch_any<double>(op, x, y, trace_pos, s);
 }
-hipError_t launch_apply_f32(const DevOperator& op, const float* x, float* y, int64_t trace_pos, hipStream_t s,
-                            bool project) {
-  return launch_any<float>(op, x, y, trace_pos, s, project);
+hipError_t launch_apply_f32(const DevOperator& op, const float* x, float* y, int64_t trace_pos, hipStream_t s) {
+  return launch_any<float>(op, x, y, trace_pos, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -461,7 +418,7 @@ hipError_t launch_apply_bicg_f64(const DevOperator& op, double* x, double* y, hi
   if (hipError_t e = hipGetLastError()) return e;
   DevOperator o = op;
   o.trace_elem = 0;   // y(1,1) of tier 0 = tr rho0 (calc_ax_bicg_omp.f90:321-324)
-  if (hipError_t e = launch_any<double>(o, x, y, 0, s, false)) return e;
+  if (hipError_t e = launch_any<double>(o, x, y, 0, s)) return e;
   hipLaunchKernelGGL(k_bicg_lower, dim3((d * d + 255) / 256), dim3(256), 0, s, d, y);
   return hipGetLastError();
 }
@@ -472,7 +429,7 @@ hipError_t launch_apply_transpose_bicg_f64(const DevOperator& op, double* w, dou
   if (hipError_t e = hipGetLastError()) return e;
   DevOperator o = op;
   o.trace_elem = 0;   // w(1,1) is the trace row's dual: kept out of L^T, added to the diagonal of z0
-  if (hipError_t e = launch_any<double>(o, w, z, 0, s, false)) return e;
+  if (hipError_t e = launch_any<double>(o, w, z, 0, s)) return e;
   hipLaunchKernelGGL(k_bicg_fold, dim3((d * d + 255) / 256), dim3(256), 0, s, d, z);
   return hipGetLastError();
 }

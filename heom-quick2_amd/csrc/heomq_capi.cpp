@@ -192,8 +192,7 @@ void fill_op(heomq_ctx* c, OperatorTables& t, const DevBuf& rec, bool transposed
   o.d = c->d;
   o.hsign = hsign;
   o.transposed = transposed;
-  o.parity = c->parity.as<int8_t>();
-  o.tb = c->tb;
+  o.n_heavy = c->L >= 1 ? c->first[c->L] : c->N;
   o.light_max = t.light_max;
   o.trace_elem = c->d * c->d - 1;
 }
@@ -1229,7 +1228,7 @@ int heomq_ctx_create(const heomq_model* h, int device, heomq_ctx** out) {
   HIPCHECK(upload(c->fwd.ent, entf));
   HIPCHECK(upload(c->trn.rowptr, rowt));
   HIPCHECK(upload(c->trn.ent, entt));
-  for (int64_t g = m.L >= 1 ? m.first[m.L] : m.N; g < m.N; ++g) {
+  for (int64_t g = m.L >= 1 ? m.first[m.L] : m.N; g < m.N; ++g) {   // the top tier: DevOperator::n_heavy on
     c->fwd.light_max = std::max<int>(c->fwd.light_max, (int)(rowf[g + 1] - rowf[g]));
     c->trn.light_max = std::max<int>(c->trn.light_max, (int)(rowt[g + 1] - rowt[g]));
   }
@@ -1237,17 +1236,6 @@ int heomq_ctx_create(const heomq_model* h, int device, heomq_ctx** out) {
   build_opmap(m, map);
   HIPCHECK(upload(c->opmap, map));
   if (int rc = upload_coefs(c.get(), m)) return rc;
-  {
-    std::vector<int8_t> par(m.d);
-    for (int i = 0; i < m.d; ++i) {
-      int ne = 0, v = i;
-      for (int o = 0; o < m.norbs; ++o, v /= 4) ne += (v % 4 == 1) + (v % 4 == 2) + 2 * (v % 4 == 3);
-      par[i] = (int8_t)(ne & 1);
-    }
-    HIPCHECK(upload(c->parity, par));
-    c->tb.ntier = m.L + 1;
-    for (int n = 0; n <= m.L + 1 && n < 12; ++n) c->tb.first[n] = m.first[n];
-  }
   fill_op(c.get(), c->fwd, c->rec, false, -1.0);
   fill_op(c.get(), c->trn, c->rec, true, +1.0);
   // derivative operator shares the forward entries; records/H/gamma set per call

@@ -126,7 +126,6 @@ struct heomq_ctx {
   std::vector<int> sec_nnz_h, fock_n, fock_s;
   std::vector<int64_t> poff_h;       // packed offset of each ADO (N + 1)
   std::vector<uint16_t> psec_h;      // sector of each ADO
-  DevBuf parity;                     // electron-number parity of each Fock state
   // symmetry-packed layout (solver path)
   DevBuf p_off, p_sec, p_elems, p_pos, p_block, p_lblock, p_entf, p_entt, p_hrow, p_hq, p_hc, p_maps;
   DevBuf p_hq_ell, p_hc_ell, p_lnz;
@@ -139,7 +138,6 @@ struct heomq_ctx {
   bool cons_n = true, cons_s = true;
   void* pinned = nullptr;            // small pinned host buffer for scalar read-back
   double* scratch_dev = nullptr;     // this device's address of the static scratch (no-alloc entry point)
-  heomq::TierBounds tb{};
   // Solves asked for on the null stream run on this non-blocking stream (the
   // null stream cannot be captured into a graph).
   hipStream_t solve_stream = nullptr;

@@ -25,12 +25,6 @@ struct DevRec {
   int32_t pad0, pad1;
 };
 
-// First ADO of each tier (for tier-dependent projections inside kernels).
-struct TierBounds {
-  int64_t first[12];   // first[ntier] = N
-  int ntier;
-};
-
 // Device tables of one operator (forward or transposed).
 struct DevOperator {
   int64_t n_ado = 0;
@@ -46,8 +40,7 @@ struct DevOperator {
   int d = 0;
   double hsign = -1.0;               // coefficient of i in hsign*i*(HX - XH)
   bool transposed = false;
-  const int8_t* parity = nullptr;    // electron-number parity of each Fock state [d]
-  TierBounds tb{};
+  int64_t n_heavy = 0;               // ADOs below the top tier (the only tier of a tier-0 hierarchy counts as one below)
   int light_max = 1;                 // most couplings of a top-tier ADO (>= 1)
   int trace_elem = 0;                // element (i + j*d) of the trace-row ADO the trace row replaces:
                                      // d*d - 1 (TFQMR convention) or 0 (BiCG convention)
@@ -242,13 +235,10 @@ hipError_t launch_herm_packed(const DevPacked& op, T* x, hipStream_t s);
 // y = A x.  trace_pos >= 0: apply the trace row at element (d-1, d-1) of ADO
 // trace_pos (forward: overwrite with tr x0; transposed: treat that element
 // of x as zero and add it to the diagonal of output block 0).
-// project = true: the output is projected onto the physical sector (elements
-// with parity(i) + parity(j) + tier odd are zeroed, the tier-0 block is
-// Hermitianised); the solvers iterate with this projected operator.
 hipError_t launch_apply_f64(const DevOperator& op, const double* x, double* y,
-                            int64_t trace_pos, hipStream_t s, bool project = false);
+                            int64_t trace_pos, hipStream_t s);
 hipError_t launch_apply_f32(const DevOperator& op, const float* x, float* y,
-                            int64_t trace_pos, hipStream_t s, bool project = false);
+                            int64_t trace_pos, hipStream_t s);
 
 // BiCG convention (bicg/calc_ax_bicg_omp.f90, calc_atrx_bicg_omp.f90).  Forward:
 // x's tier 0 is rebuilt in place from its lower triangle, y = L x, y(1,1) of

@@ -24,7 +24,7 @@ using namespace heomq;
 namespace {
 
 template <typename T>
-hipError_t apply_T(heomq_ctx* c, bool trans, const T* x, T* y, int64_t tpos, hipStream_t s, bool proj);
+hipError_t apply_T(heomq_ctx* c, bool trans, const T* x, T* y, int64_t tpos, hipStream_t s);
 // prec: 0 none; 1 left Jacobi scaling inside the apply; 2 left block-Jacobi
 // preconditioning y <- (shift - S_K)^-1 y per ADO after the apply (FP64
 // forward operator only; scratch holds the eigenbasis coefficients)
@@ -85,20 +85,19 @@ hipError_t precond_rhs(heomq_ctx* c, const float* b, float* y, float*, hipStream
   jc.ejac = c->prec_shift;
   return launch_jacobi_ado_f32(c->pfwd, jc, b, y, st);
 }
-// Solvers iterate with the projected operator Pi*A (Pi: parity sectors +
-// Hermitian tier 0).  A maps range(Pi) into itself and the physical steady
-// state is its unique solution there, so every Krylov vector stays physical
-// and round-off in the operator's non-physical null directions is removed at
-// every apply.  For the adjoint, (Pi A Pi)^T = Pi A^T Pi.
+// On packed vectors the solvers iterate with the projected operator Pi*A (Pi:
+// the symmetry sectors + Hermitian tier 0).  A maps range(Pi) into itself and
+// the physical steady state is its unique solution there, so every Krylov
+// vector stays physical and round-off in the operator's non-physical null
+// directions is removed at every apply.  For the adjoint, (Pi A Pi)^T =
+// Pi A^T Pi.  On dense vectors they iterate with the plain operator:
 template <>
-hipError_t apply_T<double>(heomq_ctx* c, bool trans, const double* x, double* y, int64_t tpos, hipStream_t s,
-                           bool proj) {
-  return launch_apply_f64(trans ? c->trn.op : c->fwd.op, x, y, tpos, s, proj);
+hipError_t apply_T<double>(heomq_ctx* c, bool trans, const double* x, double* y, int64_t tpos, hipStream_t s) {
+  return launch_apply_f64(trans ? c->trn.op : c->fwd.op, x, y, tpos, s);
 }
 template <>
-hipError_t apply_T<float>(heomq_ctx* c, bool trans, const float* x, float* y, int64_t tpos, hipStream_t s,
-                          bool proj) {
-  return launch_apply_f32(trans ? c->trn.op : c->fwd.op, x, y, tpos, s, proj);
+hipError_t apply_T<float>(heomq_ctx* c, bool trans, const float* x, float* y, int64_t tpos, hipStream_t s) {
+  return launch_apply_f32(trans ? c->trn.op : c->fwd.op, x, y, tpos, s);
 }
 
 int64_t tpos_of(const heomq_ctx* c, int trace) {
@@ -258,11 +257,11 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
   // on the unscaled trace row).
   auto Ait = [&](const T* in, T* out) -> hipError_t {
     return mode == 1 ? apply_packed_T<T>(c, trans, in, out, tpos >= 0, st, prec, W.pt)
-                     : apply_T<T>(c, trans, in, out, tpos, st, false);
+                     : apply_T<T>(c, trans, in, out, tpos, st);
   };
   auto A0 = [&](const T* in, T* out) -> hipError_t {
     return mode == 1 ? apply_packed_T<T>(c, trans, in, out, tpos >= 0, st, 0)
-                     : apply_T<T>(c, trans, in, out, tpos, st, false);
+                     : apply_T<T>(c, trans, in, out, tpos, st);
   };
   if (prec == 2) {
     if (mode != 1 || trans || !W.pt || !W.bp || (sizeof(T) != sizeof(double) && c->pjac.ado_blocks <= 0))

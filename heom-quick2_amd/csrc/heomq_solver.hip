@@ -744,40 +744,6 @@ __global__ void k_rk4_stage(int64_t n2, int first, double2* __restrict__ x, doub
   }
 }
 
-// Projection onto the physical sector: zero the elements a tier-n ADO cannot
-// hold (parity(i) + parity(j) + n odd) and Hermitianise the tier-0 block.
-template <typename T>
-__global__ void k_project_parity(int64_t nado, int d, T* __restrict__ x, const int8_t* __restrict__ par,
-                                 TierBounds tb) {
-  const int64_t dd = (int64_t)d * d;
-  GRID_LOOP(idx, nado * dd) {
-    const int64_t a = idx / dd;
-    const int e = (int)(idx - a * dd);
-    const int i = e % d, j = e / d;
-    int n = 0;
-    while (n + 1 < tb.ntier && tb.first[n + 1] <= a) ++n;
-    if ((par[i] + par[j] + n) & 1) {
-      x[2 * idx] = 0;
-      x[2 * idx + 1] = 0;
-    }
-  }
-}
-
-template <typename T>
-__global__ void k_hermitize0(int d, T* __restrict__ x) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= d * d) return;
-  const int i = e % d, j = e / d;
-  if (i > j) return;
-  const int t = j + i * d;
-  const T re = (T)0.5 * (x[2 * e] + x[2 * t]);
-  const T im = (T)0.5 * (x[2 * e + 1] - x[2 * t + 1]);
-  x[2 * e] = re;
-  x[2 * e + 1] = im;
-  x[2 * t] = re;
-  x[2 * t + 1] = -im;
-}
-
 // Scalar state reset on the device (no host staging of pageable memory).
 // Problems p < nprob with mask[p] != 0 (every problem if mask is null) are set
 // up for a (re)start: scalars cleared, flag = kInitRequested.  Problems left
@@ -942,16 +908,6 @@ hipError_t vec_axpy_f32_to_f64(hipStream_t st, int64_t n, double* x, const float
   L1(k_axpy_f32_to_f64, n, x, dx, alpha);
   return hipGetLastError();
 }
-template <typename T>
-hipError_t vec_project(hipStream_t st, int64_t nado, int d, T* x, const int8_t* par, const TierBounds& tb,
-                       bool hermitian) {
-  L1((k_project_parity<T>), nado, d, x, par, tb);
-  if (hermitian) hipLaunchKernelGGL((k_hermitize0<T>), dim3((d * d + 255) / 256), dim3(256), 0, st, d, x);
-  return hipGetLastError();
-}
-template hipError_t vec_project<double>(hipStream_t, int64_t, int, double*, const int8_t*, const TierBounds&, bool);
-template hipError_t vec_project<float>(hipStream_t, int64_t, int, float*, const int8_t*, const TierBounds&, bool);
-
 hipError_t tfq_reset(hipStream_t st, TfqmrScal* s, double target, const int32_t* mask, int nprob, bool fresh,
                      uint64_t first_seed) {
   hipLaunchKernelGGL(k_tfq_reset, dim3((nprob + 63) / 64), dim3(64), 0, st, s, target, mask, nprob, fresh ? 1 : 0,

@@ -80,10 +80,6 @@ hipError_t bicg_update(hipStream_t, int64_t n, double* x, const double* d, doubl
 hipError_t bicg_dirs(hipStream_t, int64_t n, const double* r, const double* s, double* d, double* f,
                      const BicgScal* sc);
 
-template <typename T>
-hipError_t vec_project(hipStream_t, int64_t nado, int d, T* x, const int8_t* par, const TierBounds& tb,
-                       bool hermitian);
-
 // One TFQMR iteration (Freund 1993) is: tfq_step1, A y2 -> u2, tfq_step2,
 // A w -> aw, tfq_v.  The operator is applied to w rather than to y1 = w +
 // beta y2 (A y1 = aw + beta u2), so y1 and u1 = A y1 are formed inside

@@ -1,7 +1,8 @@
 """The dense apply's heavy / light split at its edges: the shallowest
 hierarchies, ADO counts that leave the last light group ragged, and a top tier
 whose couplings exceed what one light group stages (more than 8 per ADO at
-d = 4: nine tiers, which only the reference's own arrays hold), against the oracle's dense apply and transpose."""
+d = 4: nine tiers, and twelve, which only the reference's own arrays hold), against the oracle's dense apply and
+transpose."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,7 @@ from ref_arrays import reference_arrays
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("model,nk,ntop", [("siam", 1, 1), ("siam", 2, 2), ("siam", 1, 9), ("siam", 3, 3),
+@pytest.mark.parametrize("model,nk,ntop", [("siam", 1, 1), ("siam", 2, 2), ("siam", 1, 9), ("siam", 1, 12), ("siam", 3, 3),
                                            ("dqd", 1, 1), ("dqd", 1, 2)])
 def test_dense_apply_split(model, nk, ntop):
     import torch
