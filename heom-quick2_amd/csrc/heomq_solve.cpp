@@ -274,12 +274,6 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
     if constexpr (std::is_same<T, double>::value) return mode == 1 && tfq_fusable(c, trans, tpos >= 0, prec);
     return false;
   };
-  if (fuse_ok()) {   // captured chunks hold the buffer's address: a new buffer retires them
-    const DevPacked op = fused_operator(c, trans, prec);
-    const void* before = c->partial_apply.p;
-    HIPCHECK(c->partial_apply.alloc(sizeof(double) * tfq_fused_sums(std::max(apply_jac_blocks(op), apply_blocks(op)))));
-    if (c->partial_apply.p != before) c->drop_graphs();
-  }
   TfqmrScal* s = c->scal.as<TfqmrScal>();
   double* part = c->partial.as<double>();
   double* red = c->red.as<double>();
@@ -346,7 +340,14 @@ int tfqmr_run(heomq_ctx* c, T* x, const T* b, const Work<T>& W, int64_t n, bool 
     int no_progress = 0;
     double last_check = rr;
     // the fused iteration leaves x one deferred update behind: flush() before x is read
-    const int fused = fuse_ok() && c->partial_apply.p ? (tpos >= 0 ? 1 : 0) : -1;
+    int fused = -1;
+    if (fuse_ok()) {   // captured chunks hold the sums' address: a new buffer retires them
+      const DevPacked op = fused_operator(c, trans, prec);
+      const void* before = c->partial_apply.p;
+      HIPCHECK(c->partial_apply.alloc(sizeof(double) * tfq_fused_sums(std::max(apply_jac_blocks(op), apply_blocks(op)))));
+      if (c->partial_apply.p != before) c->drop_graphs();
+      fused = tpos >= 0 ? 1 : 0;
+    }
     rs.fused = rs.fused || fused >= 0;
     auto flush = [&]() -> hipError_t {
       if constexpr (std::is_same<T, double>::value)

@@ -120,3 +120,27 @@ def test_fused_iteration_steady_state_against_the_oracle(name):
     assert st2["status"] == 0
     assert ((x2 - x).abs().max() / x.abs().max()).item() <= 1e-9
     ctx.close()
+
+
+def test_stalled_unfused_preconditioner_goes_on_fused():
+    # block Jacobi without the sector-batched top tier runs unfused; a
+    # tolerance below the residual's floor stalls it, and the solve goes on
+    # with the plain operator's fused iteration, whose sums need more room
+    # than the sparse solve before it (a pattern without the top tier) left
+    def model(ntop):
+        return heomq.Model(heomq.siam(nk=4, ntop=ntop, V=0.3, T=0.2, lscale=True))
+    m = model(3)
+    ref, _ = heomq.Context(m).solve_steady(tol=1e-12)
+    ctx = heomq.Context(m)
+    nnz, ind, irow, icol = (a.copy() for a in m.spa_pattern())
+    nnz[model(2).N:] = 0
+    ind[model(2).N:] = 0
+    ctx.set_spa_pattern(nnz, ind, irow[:nnz.sum()], icol[:nnz.sum()])
+    _, st = ctx.solve_steady_spa(tol=1e-10)
+    assert st["status"] == 0
+    ctx.set_apply_form(0, 0)
+    ctx.set_precond(2)
+    x, st = ctx.solve_steady(tol=1e-19, maxiter=20000, raise_on_fail=False)
+    print(st, flush=True)
+    assert st["status"] == heomq._lib.NOT_CONVERGED and st["fused_iteration"]
+    assert ((x - ref).abs().max() / ref.abs().max()).item() <= 1e-9
