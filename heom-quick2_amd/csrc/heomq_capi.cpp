@@ -642,6 +642,16 @@ int build_packed_host(const Model& m, const std::vector<int64_t>& rowf, const st
 }
 void set_apply_form(heomq_ctx* c, int w, int form);
 
+// The heavy rows of the fused preconditioned launch where nobody chose a form:
+// grouped while the heavy workgroups fit the chip's 256 compute units at once,
+// where the launch waits for the longest of them, sliced above, where their
+// summed work counts.  Microseconds per iteration of the two-impurity solve,
+// grouped against sliced: 42.5 / 44.0 at M = 112, L = 2 (57 heavy ADOs), 40.1 /
+// 40.0 at M = 64, L = 2; 70.0 / 69.5 at M = 64, L = 3 (1105), 149.5 / 146.8 at
+// M = 96, 213.8 / 208.5 at M = 112 (3361).
+constexpr int64_t kJacGroupedHeavy = 256;
+uint16_t jac_default_sliced(int64_t n_heavy) { return n_heavy > kJacGroupedHeavy ? 1 : 0; }
+
 int build_packed(heomq_ctx* c, const Model& m, const std::vector<int64_t>& rowf, const std::vector<DevEntry>& entf,
                  const std::vector<int64_t>& rowt, const std::vector<DevEntry>& entt) {
   PackedHost ph;
@@ -713,6 +723,7 @@ int build_packed(heomq_ctx* c, const Model& m, const std::vector<int64_t>& rowf,
     // HEOMQ_APPLY_FORM forces one.
     const char* form = std::getenv("HEOMQ_APPLY_FORM");
     set_apply_form(c, w, form ? std::atoi(form) : (c->heavy_wave_ok ? 6 : (w == 0 ? 3 : 2)));
+    if (!form) p.jac_sliced = jac_default_sliced(ph.n_heavy);
   }
   return HEOMQ_OK;
 }
@@ -733,6 +744,7 @@ void set_apply_form(heomq_ctx* c, int w, int form) {
   p.lt_off = sector ? c->p_ltoff.as<int32_t>() : nullptr;
   p.lt_id = sector ? c->p_ltados.as<int32_t>() : nullptr;
   p.lt_ent = sector ? (w == 0 ? c->p_ltent_f : c->p_ltent_t).as<DevEntryP>() : nullptr;
+  p.jac_sliced = 0;   // a chosen form is the fused preconditioned launch's too
   c->apply_form[w] = (grouped ? 1 : 0) | (sector ? 2 : 0) | (wave ? 4 : 0);
 }
 
@@ -894,6 +906,7 @@ int build_spa_operator(heomq_ctx* c, const int32_t* nnz_spa, const std::vector<i
   p.heavy_wave = ph.n_heavy > 1 ? 1 : 0;   // the pattern's heavy ADOs all small: one wave each
   for (int64_t a = 1; a < ph.n_heavy && p.heavy_wave; ++a)
     if (ph.off[a + 1] - ph.off[a] > kHeavyWaveMaxNnz) p.heavy_wave = 0;
+  p.jac_sliced = jac_default_sliced(ph.n_heavy);
   so.op = p;
   if (int rc = build_spa_h(c)) return rc;
   so.trace_slot = so.pos_h[(size_t)ph.sec[0] * dd + (d - 1) + (size_t)(d - 1) * d];

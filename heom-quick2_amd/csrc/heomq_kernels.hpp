@@ -166,7 +166,10 @@ struct DevPacked {
   // 1: ADOs 1 .. n_heavy - 1 run one wave each, four per workgroup (sectors
   // of at most 16 elements; ADO 0 keeps its own workgroup for the tier-0
   // fix-up)
-  int heavy_wave = 0;
+  uint16_t heavy_wave = 0;
+  // 1: the fused preconditioned launch takes the sliced heavy rows though the
+  // plain apply takes the grouped ones
+  uint16_t jac_sliced = 0;
   // multi-shape launches: reals before this shape's first problem in x and y
   int64_t xoff = 0;
 };

@@ -1602,7 +1602,13 @@ k_apply_packed_tfq(const DevPacked op, const double* __restrict__ x, double* __r
 // ep.prev_out[k ceil(gridDim.x / 16) + blockIdx.x]; EP 2, out =
 // aw = M^-1 A w and the partial rt.aw at ep.partial[blockIdx.x].  Nothing
 // runs once the problem's flag is set.
-template <bool RU, int EP, bool WIDE>
+//
+// GROUPED: heavy ADOs with runs take the grouped rows.  Each form is a kernel of
+// its own, as of the plain apply: one kernel with both took 213.7 us per
+// iteration of the two-impurity solve (M = 112, L = 3) on grouped and 211.8 on
+// sliced rows, the sliced kernel alone takes 208.4.  The launcher picks
+// grouped where the plain apply does and jac_sliced is not set.
+template <bool RU, int EP, bool WIDE, bool GROUPED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 k_apply_packed_jac(const DevPacked op, const DevJacobi jc, const double* __restrict__ x, double* __restrict__ out,
                    int rdo, const TfqEpi ep) {
@@ -1618,12 +1624,12 @@ k_apply_packed_jac(const DevPacked op, const DevJacobi jc, const double* __restr
   so.v = make_double2(0.0, 0.0);
   so.lbase = 0;
   so.t = 0;
-  if (heavy && op.hg_off && op.hg_off[blockIdx.x + 1] > op.hg_off[blockIdx.x])
-    heavy_grouped<double, false, WIDE, true>(op, cf, x, nullptr, -1, rdo, (int)blockIdx.x, smem, false, &so);
-  else if (heavy)
-    heavy_body<double, false, WIDE, true>(op, cf, x, nullptr, -1, rdo, (int)blockIdx.x, smem, false, &so);
-  else
+  if (!heavy)
     light_sector<double, false, WIDE, true>(op, cf, x, nullptr, -1, (int)(blockIdx.x - hb), smem, false, &so);
+  else if (GROUPED && op.hg_off[blockIdx.x + 1] > op.hg_off[blockIdx.x])
+    heavy_grouped<double, false, WIDE, true>(op, cf, x, nullptr, -1, rdo, (int)blockIdx.x, smem, false, &so);
+  else
+    heavy_body<double, false, WIDE, true>(op, cf, x, nullptr, -1, rdo, (int)blockIdx.x, smem, false, &so);
   __syncthreads();   // the apply's LDS is free from here
   double2* xw = reinterpret_cast<double2*>(smem);
   double2* tw = xw + 256;
@@ -2003,8 +2009,14 @@ static hipError_t launch_jac(const DevPacked& op, const DevJacobi& jc, const dou
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, op, jc, x, y, r, ep);
     return hipGetLastError();
   };
-  if (op.wide) return jc.u_real ? go(k_apply_packed_jac<true, EP, true>) : go(k_apply_packed_jac<false, EP, true>);
-  return jc.u_real ? go(k_apply_packed_jac<true, EP, false>) : go(k_apply_packed_jac<false, EP, false>);
+  auto pick = [&](auto ru, auto wide) {
+    constexpr bool RU = decltype(ru)::value, W = decltype(wide)::value;
+    return op.hg_off && !op.jac_sliced ? go(k_apply_packed_jac<RU, EP, W, true>) : go(k_apply_packed_jac<RU, EP, W, false>);
+  };
+  using No = std::false_type;
+  using Yes = std::true_type;
+  if (op.wide) return jc.u_real ? pick(Yes{}, Yes{}) : pick(No{}, Yes{});
+  return jc.u_real ? pick(Yes{}, No{}) : pick(No{}, No{});
 }
 
 hipError_t launch_apply_packed_jac(const DevPacked& op, const DevJacobi& jc, const double* x, double* y, bool rdo,

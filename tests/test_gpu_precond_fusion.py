@@ -144,3 +144,47 @@ def test_stalled_unfused_preconditioner_goes_on_fused():
     print(st, flush=True)
     assert st["status"] == heomq._lib.NOT_CONVERGED and st["fused_iteration"]
     assert ((x - ref).abs().max() / ref.abs().max()).item() <= 1e-9
+
+
+@pytest.mark.parametrize("name,rows", [("dqd_nk2_L2", 3), ("dqd_nk2_L3", 2)])
+def test_fused_launch_takes_its_own_heavy_rows(name, rows):
+    # by default the plain apply takes the grouped heavy rows (form 3); the
+    # fused launch takes them while the heavy ADOs are few (25 here at L = 2)
+    # and the sliced ones above (589 at L = 3), bit for bit those forms' own
+    # fused launch; a chosen form holds for both
+    import torch
+    ctx = heomq.Context(heomq.Model(CASES[name][0]()))
+    assert ctx.apply_form()[0] == 3
+    g = torch.Generator(device="cuda:0").manual_seed(7)
+    xp = torch.view_as_complex(torch.randn(ctx.packed_zeros().numel(), 2, generator=g, device="cuda:0",
+                                           dtype=torch.float64))
+    ctx.set_precond(2, 0.5)
+    y = ctx.apply_packed_precond(xp, form=4)
+    got = {}
+    for form in (2, 3):
+        ctx.set_apply_form(form, 2)
+        got[form] = ctx.apply_packed_precond(xp, form=4)
+        two = ctx.apply_packed_precond(xp, form=1)
+        assert ((got[form] - two).abs().max() / two.abs().max()).item() <= 1e-13
+    assert torch.equal(y, got[rows]) and not torch.equal(got[2], got[3])
+
+
+@pytest.mark.parametrize("name", ["dqd_nk2_L2", "dqd_nk2_L3"])
+@pytest.mark.parametrize("form", [None, 3])
+def test_fused_block_jacobi_iteration_on_grouped_rows(name, form):
+    pf, of = CASES[name]
+    ctx = heomq.Context(heomq.Model(pf()))
+    o = O.Model(of())
+    if form is not None:
+        ctx.set_apply_form(form, 2)
+    x, st = ctx.solve_steady(tol=1e-12)
+    assert st["precond"] == 2 and st["fused_iteration"]
+    xs = O.from_fortran(x.cpu().numpy())
+    e = np.zeros_like(xs)
+    e[0, o.d - 1, o.d - 1] = 1.0
+    r = e - O.physical_projection(o, O.apply(o, xs, trace_row="rdo"))
+    assert np.abs(r).max() <= 1e-10
+    ctx.set_precond_fusion(False)
+    x5, st5 = ctx.solve_steady(tol=1e-12)
+    assert not st5["fused_iteration"]
+    assert ((x - x5).abs().max() / x5.abs().max()).item() <= 1e-9
