@@ -1310,7 +1310,7 @@ int heomq_ctx_autotune(heomq_ctx* c, int reps, int32_t* forms, double* times_us)
       const DevPacked& op = w == 0 ? c->pfwd : c->ptrn;
       auto one = [&]() -> hipError_t {
         if (w == 1 || !prec_fwd) return launch_apply_packed_f64(op, xb.as<double>(), yb.as<double>(), true, st);
-        if (c->fuse_precond && apply_jac_fusable(op, jc))
+        if (c->fuse_precond && apply_jac_preferred(op, jc))
           return launch_apply_packed_jac(op, jc, xb.as<double>(), yb.as<double>(), true, st);
         if (hipError_t e = launch_apply_packed_f64(op, xb.as<double>(), tb.as<double>(), true, st)) return e;
         return launch_jacobi_1k(op, jc, tb.as<double>(), yb.as<double>(), false, st);

@@ -333,10 +333,11 @@ hipError_t launch_jacobi_1k(const DevPacked& op, const DevJacobi& jc, const doub
                             hipStream_t s);
 constexpr int kJacobiWindow = 384;    // LDS window of the one-kernel form (complex elements); d <= 16 needs <= 328
 // y = M^-1 (Pi A x), the block-Jacobi-preconditioned forward apply, in one
-// launch (no A x in HBM).  Needs the sector-batched top tier and a
-// workgroup per heavy ADO (apply forms 2 and 3), one problem, no Jacobi
-// scaling, d <= 16 and the ADO-aligned inverse's tables.
+// launch (no A x in HBM).  Needs the sector-batched top tier (apply forms 2,
+// 3, 6 and 7), one problem, no Jacobi scaling, d <= 16 and the ADO-aligned
+// inverse's tables.  apply_jac_preferred: and faster than the two launches.
 bool apply_jac_fusable(const DevPacked& op, const DevJacobi& jc);
+bool apply_jac_preferred(const DevPacked& op, const DevJacobi& jc);
 hipError_t launch_apply_packed_jac(const DevPacked& op, const DevJacobi& jc, const double* x, double* y, bool rdo,
                                    hipStream_t s);
 

@@ -1997,8 +1997,20 @@ hipError_t launch_jacobi_ado_f32(const DevPacked& op, const DevJacobi& jc, const
 }
 
 bool apply_jac_fusable(const DevPacked& op, const DevJacobi& jc) {
-  return op.lt_blk != nullptr && !op.heavy_wave && !op.transposed && op.precond == 0 &&
-         op.nprob == 1 && op.n_heavy > 0 && op.d <= 16 && jc.ado_blocks > 0 && jc.desc != nullptr;
+  return op.lt_blk != nullptr && !op.transposed && op.precond == 0 && op.nprob == 1 && op.n_heavy > 0 &&
+         op.d <= 16 && jc.ado_blocks > 0 && jc.desc != nullptr;
+}
+
+// The fused launch takes a workgroup per heavy ADO, whatever the plain apply
+// takes.  Where the plain apply runs small sectors one wave each, a workgroup
+// has most lanes idle: worth it for the launch and the vector passes it saves
+// while the heavy ADOs are few.  Microseconds per iteration, fused against wave
+// apply + inverse + vector passes, single impurity with block Jacobi: 38.2 /
+// 48.5 at 21 heavy ADOs, 41.2 / 48.6 at 1477, 52.4 / 54.3 at 2777, 72.6 / 58.2
+// at 5401, 209.7 / 123.0 at 22,001.
+constexpr int64_t kJacFuseWaveHeavy = 3072;
+bool apply_jac_preferred(const DevPacked& op, const DevJacobi& jc) {
+  return apply_jac_fusable(op, jc) && (!op.heavy_wave || op.n_heavy <= kJacFuseWaveHeavy);
 }
 
 template <int EP>

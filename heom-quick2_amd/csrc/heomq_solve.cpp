@@ -48,7 +48,7 @@ hipError_t apply_packed_T<double>(heomq_ctx* c, bool trans, const double* x, dou
   if (prec != 2) return trans ? launch_apply_packed_f64(op, x, y, rdo, s) : packed_forward(c, op, x, y, rdo, s);
   DevJacobi jc = c->pjac;
   jc.ejac = c->prec_shift;
-  if (c->fuse_precond && !c->trun.built && apply_jac_fusable(op, jc))   // one launch, no A x in HBM
+  if (c->fuse_precond && !c->trun.built && apply_jac_preferred(op, jc))   // one launch, no A x in HBM
     return launch_apply_packed_jac(op, jc, x, y, rdo, s);
   if (jacobi_one_kernel(jc)) {   // A x into the scratch, then y = M^-1 (A x) in one kernel
     if (hipError_t e = packed_forward(c, op, x, scratch, rdo, s)) return e;
@@ -151,7 +151,7 @@ bool tfq_fusable(heomq_ctx* c, bool trans, bool rdo, int prec) {
   if (off || !c->fuse_precond || c->trun.built) return false;
   const DevPacked op = fused_operator(c, trans, prec);
   if (rdo && op.trace_slot < 0) return false;
-  return prec == 2 ? !trans && apply_jac_fusable(op, c->pjac) : apply_tfq_fusable(op);
+  return prec == 2 ? !trans && apply_jac_preferred(op, c->pjac) : apply_tfq_fusable(op);
 }
 
 // Sums of the fused iteration's operator launches over na workgroups: four
@@ -958,8 +958,8 @@ int heomq_apply_packed_precond(heomq_ctx* c, const double* xp, double* yp, int t
   jc.ejac = c->prec_shift;
   if (form == 4) {
     if (c->trun.built || !apply_jac_fusable(op, jc))
-      return fail(HEOMQ_UNSUPPORTED, "the fused preconditioned apply needs a sector-batched apply form without the wave form "
-                                     "and the ADO-aligned inverse");
+      return fail(HEOMQ_UNSUPPORTED, "the fused preconditioned apply needs a sector-batched apply form and the "
+                                     "ADO-aligned inverse");
     HIPCHECK(launch_apply_packed_jac(op, jc, xp, yp, rdo, st));
     return HEOMQ_OK;
   }

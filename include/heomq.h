@@ -191,9 +191,9 @@ int heomq_ctx_set_presmooth(heomq_ctx* c, int enable);
 /* Block-Jacobi-preconditioned packed applies (the steady solve's iteration,
  * heomq_apply_packed_precond) run as one fused launch, the inverse applied to
  * each workgroup's ADOs before anything is written, when the forward apply
- * form has the sector-batched top tier and a workgroup per heavy row (enable =
- * 1, the default; the same values); 0 always runs the apply, then the
- * inverse.  The same switch lets the plain and Jacobi-scaled solver iterations
+ * form has the sector-batched top tier (forms 2, 3, 6, 7; with the wave form up
+ * to 3072 ADOs below the top tier, where it is the faster way) (enable = 1,
+ * the default; the same values); 0 always runs the apply, then the inverse.  The same switch lets the plain and Jacobi-scaled solver iterations
  * carry their vector work in the apply, and fuses each Chebyshev term of the packed
  * propagators (the apply's output folded into the recurrence and the sum,
  * one launch, the same bits).  No counterpart in the reference. */
@@ -275,8 +275,8 @@ int heomq_apply_packed_raw_f32(heomq_ctx* c, const float* xp, float* yp, int tra
  * apply, then the two-kernel transform; 3: apply, then the LDS-window kernel
  * (when every ADO range a 256-element block touches fits its LDS); 4: one
  * fused launch, the inverse applied in each apply workgroup to its whole
- * ADOs (the sector-batched apply forms without the wave form, d <= 16, the
- * ADO-aligned inverse), HEOMQ_UNSUPPORTED otherwise.  All forms
+ * ADOs (the sector-batched apply forms 2, 3, 6 and 7, d <= 16, the ADO-aligned
+ * inverse), HEOMQ_UNSUPPORTED otherwise.  All forms
  * compute the same values.  No counterpart in the reference. */
 int heomq_apply_packed_precond(heomq_ctx* c, const double* xp, double* yp, int trace, int form, void* stream);
 /* The same operator as heomq_apply_packed_precond form 1, with no allocation:

@@ -188,3 +188,28 @@ def test_fused_block_jacobi_iteration_on_grouped_rows(name, form):
     x5, st5 = ctx.solve_steady(tol=1e-12)
     assert not st5["fused_iteration"]
     assert ((x - x5).abs().max() / x5.abs().max()).item() <= 1e-9
+
+
+@pytest.mark.parametrize("nk,ntop", [(2, 3), (4, 4)])
+def test_small_sectors_keep_the_fused_block_jacobi_iteration(nk, ntop):
+    # every sector of the single impurity is small, so the plain apply takes
+    # one wave per heavy ADO; block Jacobi still has its fused launch, which
+    # the solver takes while the heavy ADOs are few (157 against 5401 here)
+    import torch
+    ctx = heomq.Context(heomq.Model(heomq.siam(nk=nk, ntop=ntop, V=0.3, U=1.5, lscale=True)))
+    ctx.set_precond(2)
+    x, st = ctx.solve_steady(tol=1e-11)
+    assert st["precond"] == 2 and st["fused_iteration"] == (ntop == 3)
+    ctx.set_precond_fusion(False)
+    x5, st5 = ctx.solve_steady(tol=1e-11)
+    assert not st5["fused_iteration"]
+    assert ((x - x5).abs().max() / x5.abs().max()).item() <= 1e-8
+    ctx.set_precond_fusion(True)
+    g = torch.Generator(device="cuda:0").manual_seed(8)
+    xp = torch.view_as_complex(torch.randn(ctx.packed_zeros().numel(), 2, generator=g, device="cuda:0",
+                                           dtype=torch.float64))
+    for form in (None, 2, 7):
+        if form is not None:
+            ctx.set_apply_form(form, form)
+        y1, y4 = (ctx.apply_packed_precond(xp, form=f) for f in (1, 4))
+        assert ((y1 - y4).abs().max() / y1.abs().max()).item() <= 1e-13
