@@ -88,6 +88,42 @@ __device__ inline void add_couplings(const Coupling<T>* cs, int stride, int nv, 
   }
 }
 
+// One coupling of KC elements (i, j0 + q dj) of a lane (d = 64), every
+// neighbour element loaded before any is used; smap as above.
+template <int D, typename T, bool TRANS, int KC>
+__device__ inline void add_coupling_elems(const Coupling<T>& c, const int8_t* smap,
+                                          const typename V2<T>::type* __restrict__ xv, int i, int j0, int dj,
+                                          int64_t trace_pos, int trace_elem, T* ar, T* ai) {
+  using V = typename V2<T>::type;
+  if (c.op == 0xff) return;   // block-uniform
+  const V* __restrict__ xn = xv + (int64_t)c.nbr * (D * D);
+  const bool zero = TRANS && c.nbr == trace_pos;
+  const int ml = smap[c.op * 2 * D + i], pl = (ml < 0 ? -ml : ml) - 1;
+  V vl[KC], vr[KC];
+  int mr[KC];
+#pragma unroll
+  for (int q = 0; q < KC; ++q) {
+    const int j = j0 + q * dj;
+    mr[q] = smap[c.op * 2 * D + D + j];
+    const int pr = (mr[q] < 0 ? -mr[q] : mr[q]) - 1;
+    const int el = c.dag ? j + pl * D : pl + j * D, er = c.dag ? pr + i * D : i + pr * D;
+    vl[q] = V{0, 0};
+    vr[q] = V{0, 0};
+    if (ml != 0 && !(zero && el == trace_elem)) vl[q] = xn[el];
+    if (mr[q] != 0 && !(zero && er == trace_elem)) vr[q] = xn[er];
+  }
+  const T cj = c.dag ? (T)-1 : (T)1, sl = ml < 0 ? (T)-1 : (T)1;
+#pragma unroll
+  for (int q = 0; q < KC; ++q) {
+    const T sr = mr[q] < 0 ? (T)-1 : (T)1;   // a zero element where there is no term
+    const T lx = sl * vl[q].x, ly = sl * cj * vl[q].y, rx = sr * vr[q].x, ry = sr * cj * vr[q].y;
+    ar[q] += c.clr * lx - c.cli * ly;
+    ai[q] += c.clr * ly + c.cli * lx;
+    ar[q] += c.crr * rx - c.cri * ry;
+    ai[q] += c.crr * ry + c.cri * rx;
+  }
+}
+
 // What a workgroup stages once: the operators' maps and, for d <= 16, H by
 // rows with the row index fastest (16 rows of one column index are
 // consecutive: no bank conflicts).
@@ -155,9 +191,15 @@ struct DenseLds {
 // the couplings in flight (4 heavy and 3 light at d = 16, 2 and 2 at d = 4)
 // are the most that keep 80 VGPRs without scratch, 6 waves per SIMD.  FP64
 // forward, with one ADO per workgroup slot and its couplings walked one by one
-// before: 1415 -> 514 us at two-impurity size (M = 112, L = 3; 962 MB, 1.9
+// before: 1415 -> 513 us at two-impurity size (M = 112, L = 3; 962 MB, 1.9
 // TB/s), 71 -> 15 us and 441 -> 216 us at the single impurity's M = 72, L = 3
-// and 4.  Ordering the heavy workgroups among the light ones by their
+// and 4.  At d = 64 a lane has 16 elements; KC of them share a walk over the
+// couplings, with 2 KC gathers in flight, and the couplings are staged once
+// where they fit.  Three orbitals, M = 48, FP64 (KC = 8) forward at L = 1 / 2 / 3:
+// 284 / 389 / 1612 us with one element at a time, 122 / 156 / 1034 us now (KC = 4:
+// 140 / 186 / 1032; KC = 16, with 500 bytes of scratch a lane: 117 / 152 / 1354);
+// FP32 (KC = 4, four workgroups per CU) 265 / 358 / 934 -> 135 / 176 / 671 us (KC =
+// 8: 119 / 151 / 828).  Ordering the heavy workgroups among the light ones by their
 // neighbours' place gave 597 against 622 us at an earlier stage, for a table
 // built per context: not kept.
 template <int D, typename T, bool TRANS>
@@ -168,7 +210,8 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
   constexpr int LANES = E < 256 ? E : 256;
   constexpr int EPT = E / LANES;
   constexpr int APB = 256 / LANES;   // ADOs of a light group, slices of a heavy ADO
-  constexpr int U = EPT > 1 ? 1 : (D == 4 ? 2 : 4), UL = EPT > 1 ? 1 : (D == 4 ? 2 : 3);   // couplings in flight, heavy and light
+  constexpr int U = D == 4 ? 2 : 4, UL = D == 4 ? 2 : 3;   // couplings in flight, heavy and light
+  constexpr int KC = EPT > 1 ? (sizeof(T) == 8 ? 8 : 4) : 1;   // d = 64: elements of a lane in flight instead
   __shared__ V xs[EPT == 1 ? 512 : E];
   __shared__ DenseLds<D> tab;
   __shared__ Coupling<T> s_c[kStage];
@@ -189,14 +232,36 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
     }
     const T gr = (T)op.gam[2 * a], gi = (T)op.gam[2 * a + 1];
     const int64_t p0 = op.rowptr[a], p1 = op.rowptr[a + 1];
-    for (int k = 0; k < EPT; ++k) {
-      const int e = lane + k * LANES;
+    auto stage_heavy = [&](int64_t q0) {
+      const int n = (int)(p1 - q0 < kStage ? p1 - q0 : kStage);
+      __syncthreads();   // the previous stage is read
+      if (tid < n) s_c[tid] = to_coupling<T>(op, op.ent[q0 + tid]);
+      __syncthreads();
+      return n;
+    };
+    if constexpr (EPT > 1) {
+      int n = 0;
+      for (int k0 = 0; k0 < EPT; k0 += KC) {
+        T ar[KC] = {}, ai[KC] = {};
+        for (int64_t q0 = p0; q0 < p1; q0 += kStage) {
+          if (k0 == 0 || p1 - p0 > kStage) n = stage_heavy(q0);   // one stage serves every pass where all couplings fit
+          for (int c = 0; c < n; ++c)
+            add_coupling_elems<D, T, TRANS, KC>(s_c[c], tab.smap, xv, lane % D, (lane + k0 * LANES) / D, LANES / D,
+                                                trace_pos, op.trace_elem, ar, ai);
+        }
+        if (k0 == 0) __syncthreads();   // xs is staged (also for an ADO without couplings)
+#pragma unroll
+        for (int q = 0; q < KC; ++q) {
+          const int e = lane + (k0 + q) * LANES;
+          tab.template same_tier<T>(op, xs, gr, gi, e % D, e / D, ar[q], ai[q]);
+          yv[a * E + e] = V{ar[q], ai[q]};
+        }
+      }
+    } else {
+      const int e = lane;
       T ar = 0, ai = 0;
       for (int64_t q0 = p0; q0 < p1; q0 += kStage) {
-        const int n = (int)(p1 - q0 < kStage ? p1 - q0 : kStage);
-        __syncthreads();   // the previous stage is read
-        if (tid < n) s_c[tid] = to_coupling<T>(op, op.ent[q0 + tid]);
-        __syncthreads();
+        const int n = stage_heavy(q0);
         for (int c0 = slot; c0 < n; c0 += APB * U) {
           const int nv = (n - c0 + APB - 1) / APB;
           add_couplings<D, T, TRANS, U>(s_c + c0, APB, nv < U ? nv : U, tab.smap, xv, e % D, e / D, trace_pos,
@@ -220,9 +285,7 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
         ar = xs[tid].x;
         ai = xs[tid].y;
       }
-      if (slot == 0) {
-        yv[a * E + e] = V{ar, ai};
-      }
+      if (slot == 0) yv[a * E + e] = V{ar, ai};
     }
     return;
   }
@@ -265,8 +328,29 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
     }
     V g{0, 0};
     if (active) g = V{(T)op.gam[2 * a], (T)op.gam[2 * a + 1]};
-    for (int k = 0; k < EPT; ++k) {
-      const int e = lane + k * LANES;
+    if constexpr (EPT > 1) {
+      for (int k0 = 0; k0 < EPT; k0 += KC) {
+        T ar[KC] = {}, ai[KC] = {};
+        for (int c0 = 0; c0 < light_max; c0 += per) {
+          if (per < light_max) {   // uniform
+            __syncthreads();
+            stage_light(c0);
+            __syncthreads();
+          }
+          for (int u = 0; u < per; ++u)
+            add_coupling_elems<D, T, TRANS, KC>(s_c[r * per + u], tab.smap, xv, lane % D, (lane + k0 * LANES) / D,
+                                                LANES / D, trace_pos, op.trace_elem, ar, ai);
+        }
+        if (k0 == 0) __syncthreads();   // xs is staged
+#pragma unroll
+        for (int q = 0; q < KC; ++q) {
+          const int e = lane + (k0 + q) * LANES;
+          tab.template same_tier<T>(op, xs, g.x, g.y, e % D, e / D, ar[q], ai[q]);
+          yv[a * E + e] = V{ar[q], ai[q]};
+        }
+      }
+    } else {
+      const int e = lane;
       T ar = 0, ai = 0;
       for (int c0 = 0; c0 < light_max; c0 += per) {
         if (per < light_max) {   // uniform
@@ -279,7 +363,7 @@ k_apply(const DevOperator op, const T* __restrict__ x, T* __restrict__ y, int64_
             add_couplings<D, T, TRANS, UL>(&s_c[(r * APB + slot) * per + u], 1, per - u < UL ? per - u : UL, tab.smap,
                                            xv, e % D, e / D, trace_pos, op.trace_elem, ar, ai);
       }
-      if (k == 0) __syncthreads();   // xs is staged
+      __syncthreads();   // xs is staged
       if (active) {
         tab.template same_tier<T>(op, xr + slot * E, g.x, g.y, e % D, e / D, ar, ai);
         yv[a * E + e] = V{ar, ai};

@@ -21,21 +21,21 @@ pytestmark = pytest.mark.gpu
 _cache = {}
 
 
-def params(L):
-    return O.Params(norbs=3, nspin=2, nalf=2, nmats=1, bandwidth=(10.0, 10.0),
+def params(L, nmats=1):
+    return O.Params(norbs=3, nspin=2, nalf=2, nmats=nmats, bandwidth=(10.0, 10.0),
                     linewidth=((0.1, 0.08, 0.12), (0.1, 0.08, 0.12)), temperature=(0.2, 0.2),
                     engyshift=((0.1, 0.1), (-0.1, -0.1)), ham="siam",
                     hpar=dict(eup=-0.5, edown=-0.5, uu=1.0), ntop=L)
 
 
-def setup(L):
-    if L not in _cache:
+def setup(L, nmats=1):
+    if (L, nmats) not in _cache:
         import torch
-        o = O.Model(params(L))
+        o = O.Model(params(L, nmats))
         m = heomq.Model.from_reference(**reference_arrays(o))
         ctx = heomq.Context(m)
-        _cache[L] = (o, m, ctx, torch)
-    return _cache[L]
+        _cache[L, nmats] = (o, m, ctx, torch)
+    return _cache[L, nmats]
 
 
 def to_dev(torch, x):
@@ -62,6 +62,19 @@ def test_d64_dense_apply_and_transpose(L, trace):
     w = O.seeded_ado_vector(o, 32)
     assert rel(from_dev(ctx.apply_transpose(to_dev(torch, w), trace=tr)),
                O.apply_transpose(o, w, trace_row=trace)) <= 1e-12
+
+
+def test_d64_dense_apply_of_long_rows():
+    # M = 144: tier 0's couplings exceed what a workgroup stages at once (128)
+    o, m, ctx, torch = setup(1, 5)
+    assert m.M == 144
+    x = O.seeded_ado_vector(o, 35)
+    xd = to_dev(torch, x)
+    assert rel(from_dev(ctx.apply(xd, trace=heomq.TRACE_LAST)), O.apply(o, x, trace_row="last")) <= 1e-12
+    assert rel(from_dev(ctx.apply_transpose(xd, trace=heomq.TRACE_LAST)),
+               O.apply_transpose(o, x, trace_row="last")) <= 1e-12
+    y = from_dev(ctx.apply_f32(xd.to(torch.complex64), trace=heomq.TRACE_NONE))
+    assert rel(y, O.apply(o, x, trace_row=None)) <= 2e-6
 
 
 @pytest.mark.parametrize("L", [1, 2])
