@@ -2,8 +2,8 @@
 elements) against the 64-bit ones of larger vectors, forced on the same
 layout, over models with one to many lanes per ADO, every form, both
 directions, both precisions and the Chebyshev and preconditioned epilogues;
-and the grouped rows' run splitting (one, two and four parts) against the
-oracle."""
+the grouped rows' run splitting (one, two and four parts) and the top-tier
+records of small sectors, in LDS and beyond its room, against the oracle."""
 import numpy as np
 import pytest
 
@@ -17,7 +17,7 @@ MODELS = {"siam_L1": lambda: heomq.siam(nk=1, ntop=1), "siam_L4": lambda: heomq.
 
 
 @pytest.mark.parametrize("name", list(MODELS))
-def test_wide_gathers_give_the_same_bits(name, monkeypatch):
+def test_wide_gathers_give_the_same_values(name, monkeypatch):
     import torch
     m = heomq.Model(MODELS[name]())
     narrow = heomq.Context(m)
@@ -58,3 +58,22 @@ def test_grouped_rows_match_oracle(model, nk, ntop):
         y = O.from_fortran(ctx.apply_packed(xd, trace=heomq.TRACE_RDO, transpose=transpose).cpu().numpy())
         ref = O.physical_projection(o, f(o, x, trace_row="rdo"))
         assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nk", [8, 9])
+def test_small_sector_records_match_oracle(nk):
+    # one wave per heavy ADO: a top-tier block stages the records it may use
+    # while they are at most 224 (forward M of them, transposed 3 M: 216 at M =
+    # 72, 240 at M = 80, which load theirs from memory)
+    import torch
+    ctx = heomq.Context(heomq.Model(heomq.siam(nk=nk, ntop=2, V=0.3)))
+    o = O.Model(O.siam_params(nk=nk, ntop=2, V=0.3))
+    assert ctx.apply_form() == (6, 6)
+    x = O.physical_projection(o, O.seeded_ado_vector(o, 10))
+    xp = ctx.pack(torch.from_numpy(O.to_fortran(x)).to("cuda:0"))
+    for transpose, f in ((False, O.apply), (True, O.apply_transpose)):
+        ref = O.physical_projection(o, f(o, x, trace_row="rdo"))
+        for dtype, tol in ((torch.complex128, 1e-12), (torch.complex64, 2e-6)):
+            yp = ctx.apply_packed_raw(xp.to(dtype), ctx.packed_zeros(dtype), transpose=transpose)
+            y = O.from_fortran(ctx.unpack(yp.to(torch.complex128)).cpu().numpy())
+            assert np.abs(y - ref).max() <= tol * np.abs(ref).max()
