@@ -170,7 +170,6 @@ __device__ inline void put_half(TfqmrScal* s, const Half& h) {
   s->eta = h.eta;
   s->dcoef = h.dcoef;
 }
-__device__ inline void half_step(TfqmrScal* s, double a) { put_half(s, half_of(a, s->tau, s->alpha)); }
 
 // The scalars copied word by word through registers.  (A TfqmrScal local to
 // k_step2 or k_v, read and written through its address, was given 69 and 32 KB
@@ -185,24 +184,6 @@ __device__ inline void copy_scal(const TfqmrScal* from, TfqmrScal* to) {
   for (int k = 0; k < kWords; ++k) v[k] = p[k];
 #pragma unroll
   for (int k = 0; k < kWords; ++k) q[k] = v[k];
-}
-
-// The second half step of an iteration, then rho_new = rt.w = b: the bound
-// met sets stop (the x update of the iteration still runs, k_v; the final
-// finalize then stops), rho = 0 is a breakdown.
-__device__ inline void half_step_rho(TfqmrScal* s, double a, double b) {
-  half_step(s, a);
-  s->iter += 1;
-  if (s->tau * sqrt(2.0 * s->iter + 1.0) <= s->target) {
-    s->stop = 1;
-    return;
-  }
-  if (s->rho == 0.0) {
-    s->flag = 2;
-    return;
-  }
-  s->beta = b / s->rho;
-  s->rho = b;
 }
 
 // The iteration is kept in a form that applies the operator to w instead of
@@ -404,7 +385,9 @@ __global__ void k_v(const Loc loc, const T* __restrict__ aw, const T* __restrict
   if (first) copy_scal(s_in, s_out);
   double a, b;
   fold_sum(pa, pb, a, b);
-  // half_step_rho on values
+  // the second half step, then rho_new = rt.w = b: the bound met sets stop (the
+  // x update of the iteration still runs; the final finalize then stops), rho =
+  // 0 is a breakdown
   const Half h = half_of(a, tau, alpha0);
   const bool next = !(h.tau * sqrt(2.0 * iter + 1.0) <= target);
   const bool broken = next && rho == 0.0;
@@ -545,7 +528,7 @@ __global__ void __launch_bounds__(kFoldThreads) k_tfq_fold(const double* __restr
   }
   const double a1 = v[0], sv = v[1], a2 = v[2], rw = v[3], ru = v[4], ra = v[5];
   const Half h = half_of(a1, s_tau, s_alpha);
-  // the second half step, the stop test and rho (half_step_rho on values)
+  // the second half step, the stop test and rho, as in k_v
   const Half g = half_of(a2, h.tau, s_alpha);
   const int iter = s_iter + 1;
   const bool stop = g.tau * sqrt(2.0 * iter + 1.0) <= s_target;
@@ -618,7 +601,7 @@ __global__ void k_resid(const Loc loc, const TB* __restrict__ b, const TA* __res
 
 // Phase 2: one block folds the partials in a fixed order and advances the
 // scalars (Freund 1993; Saad, Iterative Methods 7.4.2).
-enum FinalizeOp { F_INIT_R = 0, F_INIT_V, F_HALF, F_HALF_RHO, F_V, F_RESID };
+enum FinalizeOp { F_INIT_R = 0, F_INIT_V, F_V, F_RESID };
 
 
 // Block q finalizes problem q (one block for a single problem; the covered
@@ -662,12 +645,6 @@ __global__ void k_finalize(const Loc loc, int op, int nblk_uni, const double* __
       s->alpha = s->rho / a;
       s->dcoef = 0;
       s->flag = 0;
-      break;
-    case F_HALF:
-      half_step(s, a);
-      break;
-    case F_HALF_RHO:   // second half step, then rho_new = rt.w = b
-      half_step_rho(s, a, b);
       break;
     case F_V:
       if (s->stop) { s->flag = 1; break; }
