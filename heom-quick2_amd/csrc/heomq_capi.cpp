@@ -715,12 +715,14 @@ int build_packed(heomq_ctx* c, const Model& m, const std::vector<int64_t>& rowf,
     p.lt_rec0 = (uint16_t)ph.lt_rec0[w];
     p.lt_recn = (uint16_t)ph.lt_recn[w];
     // the default form: the sector-batched top tier; below it one wave per ADO
-    // where every sector is small (the single impurity: 36.8 against 89.2 us in
-    // form 2 at M = 72, L = 4, 6.8 against 8.4 at L = 3), else the grouped rows
-    // forward (two impurities, M = 112, L = 3: 50.5 against 56.2 us, 14.5 against
-    // 16.5 at M = 64) and the sliced ones transposed (52 against 53 us, 7.5
-    // against 8.1 at L = 2, 15.9 against 15.4 at M = 64).  The autotuner (heomq_ctx_autotune) picks per operator,
-    // HEOMQ_APPLY_FORM forces one.
+    // where every sector is small (the single impurity, form 6 against 2: 34.2 /
+    // 85.3 us at M = 72, L = 4, 7.8 / 16.7 at M = 40, L = 4, 6.7 / 8.3 at M = 72,
+    // L = 3), else the grouped rows forward (two impurities, form 3 against 2:
+    // 51.0 / 52.9 us at M = 112, L = 3, 34.4 / 36.3 at M = 96, 14.8 / 16.3 at M =
+    // 64, 10.4 / 11.6 at M = 112, L = 2; a Chebyshev term 62.0 / 66.1) and the
+    // sliced ones transposed (53.3 / 50.3, 36.8 / 34.9, 15.7 / 15.6, 8.5 / 7.8).
+    // The autotuner (heomq_ctx_autotune) picks per operator, HEOMQ_APPLY_FORM
+    // forces one.
     const char* form = std::getenv("HEOMQ_APPLY_FORM");
     set_apply_form(c, w, form ? std::atoi(form) : (c->heavy_wave_ok ? 6 : (w == 0 ? 3 : 2)));
     if (!form) p.jac_sliced = jac_default_sliced(ph.n_heavy);

@@ -131,7 +131,7 @@ struct DevPacked {
   int lt_u = 0;
   // slot-space tables: i(HX - XH) per sector as CSR over packed slots, and the
   // gather maps (kMapAbsent: no term) referenced by entries
-  // the same rows padded to a fixed width hell_w (slot -1 / coefficient 0 as
+  // the same rows padded to a fixed width hell_w (slot 0 with coefficient 0 as
   // padding) when every row is short: index loads then depend only on (s, t)
   int hell_w = 0;                    // 0: use the CSR form
   int hell_wp = 0;                   // hell_w rounded up to 8 (index rows are read 8 at a time)

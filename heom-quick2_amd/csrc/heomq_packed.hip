@@ -96,7 +96,8 @@ __device__ inline int2 map_at(const int2* __restrict__ maps, int map, int t) {
   if (WIDE) return maps[(int64_t)map + t];
   return *reinterpret_cast<const int2*>(reinterpret_cast<const char*>(maps) + (uint32_t)((map + t) << 3));
 }
-// t / w for t <= 256, 1 <= w <= 256 (exact: t (inv w - 65536) < 65536)
+// t / w for t <= 256, 1 <= w <= 256 (exact: t (inv w - 65536) <= 65536, with
+// equality at t = w = 256 only)
 __device__ inline int div_inv(int w) { return (int)(65536.0f * __frcp_rn((float)w)) + 1; }
 __device__ inline int div_by(int t, int inv) { return (int)(((uint32_t)t * (uint32_t)inv) >> 16); }
 
@@ -990,14 +991,16 @@ __device__ inline void light_sector(const DevPacked& op, const Coefs cf_p, const
 // top tier (dispatched first: their work per block is the longest), the rest
 // the top tier's elements, so the two phases overlap on the device.  The LDS
 // buffer allows 7 blocks per CU; the register budget is held to the same 7
-// waves per SIMD (72 VGPRs).
+// waves per SIMD (72 VGPRs; the forward FP64 kernels of forms 2 and 3 spill 28
+// bytes a lane at that, the Chebyshev ones 36).
 //
 // Bound by no one unit: at two-impurity size (M = 112, L = 3, 1.8 M elements)
 // the address units are busy 57 % of the time, the vector units 45 %, and the
 // Infinity Cache delivers 166 MB (the top tier four times); each workgroup is
-// a chain of five or six dependent loads.  FP64 forward 58.7 us (form 2, the
-// former default) -> 50.5 us (form 3), transposed 64.6 -> 52.3; single impurity
-// M = 72, L = 4: 83.4 us (form 2) -> 34.7 us (form 6).
+// a chain of five or six dependent loads.  Launches one after another, both
+// builds on one card: FP64 forward 54.0 us (form 2, the maps in slots, entries
+// gathered per lane) -> 51.0 us (form 3; form 2 52.9), transposed 61.8 -> 50.3
+// (form 2); single impurity M = 72, L = 4: 82.1 us (form 2) -> 34.2 us (form 6).
 constexpr size_t kApplySmem1 = kGSmem > kLSmem ? kGSmem : kLSmem;
 constexpr size_t kApplySmem = kApplySmem0 > kApplySmem1 ? kApplySmem0 : kApplySmem1;
 
@@ -1572,8 +1575,8 @@ __device__ inline void tfq_partials(double r0, double r1, double r2, const TfqEp
 // its outputs (TfqPut): k_step2 and the v update of k_v and their launches are
 // gone from the iteration, as in the preconditioned one below (single impurity,
 // 37,012 elements: 35.4 -> 27.1 us of kernels per iteration; 8.0 and 7.3 us for
-// the two applies with their epilogues against 7.2 without).  6 waves per SIMD:
-// 72 VGPRs spilled 44 bytes per lane.
+// the two applies with their epilogues against 7.2 without).  6 waves per SIMD
+// (80 VGPRs): the forward kernels of form 6 spill 20 bytes a lane, 44 at 7 waves.
 template <bool TRANS, int FORM, int KIND>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 k_apply_packed_tfq(const DevPacked op, const double* __restrict__ x, double* __restrict__ y, int64_t zero_at, int rdo,

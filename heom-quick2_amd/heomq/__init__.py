@@ -478,7 +478,7 @@ class Context:
 
     def set_precond_fusion(self, enable: bool):
         """Block-Jacobi-preconditioned applies as one fused launch where the
-        apply form allows it (the same bits as the two kernels), and solver
+        apply form allows it (the same values as the two kernels), and solver
         iterations with their vector work in the operator launches (default
         on)."""
         check(lib().heomq_ctx_set_precond_fusion(self._h, int(enable)))
