@@ -1607,9 +1607,9 @@ k_apply_packed_tfq(const DevPacked op, const double* __restrict__ x, double* __r
 // runs once the problem's flag is set.
 //
 // GROUPED: heavy ADOs with runs take the grouped rows.  Each form is a kernel of
-// its own, as of the plain apply: one kernel with both took 213.7 us per
+// its own, as of the plain apply: one kernel with both took 214.4 us per
 // iteration of the two-impurity solve (M = 112, L = 3) on grouped and 211.8 on
-// sliced rows, the sliced kernel alone takes 208.4.  The launcher picks
+// sliced rows, kernels of their own 213.8 and 208.5.  The launcher picks
 // grouped where the plain apply does and jac_sliced is not set.
 template <bool RU, int EP, bool WIDE, bool GROUPED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))

@@ -766,8 +766,9 @@ class Context:
                      raise_on_fail=True):
         """TFQMR steady state on the device; returns (x, stats dict): iters,
         applies, relres, seconds, status, precond (the left preconditioner
-        the iteration ended with) and fused_iteration (iterations ran with
-        their vector work in the operator launches)."""
+        the solve took; one that stalls is dropped on the way) and
+        fused_iteration (iterations ran with their vector work in the operator
+        launches)."""
         t = self.torch
         x = self.initial_guess() if x is None else x
         stats = np.zeros(_lib.STATS_LEN)

@@ -322,8 +322,8 @@ int heomq_calcderiv(heomq_ctx* c, const double* rhotmp_host, double* rhorhs_host
  * ||b - A x||_2 <= tol * ||b||_2 on the (Re, Im) vector.  transpose = 1 solves
  * with A^T (the adjoint solve).  b may be NULL (then b = e_trace).
  * stats (HEOMQ_STATS_LEN): [0] iterations, [1] applies, [2] final relative
- * residual, [3] seconds, [4] the left preconditioner the iteration ended
- * with (0 none, 1 Jacobi scaling, 2 block Jacobi), [5] length of the real
+ * residual, [3] seconds, [4] the left preconditioner the solve took (0 none,
+ * 1 Jacobi scaling, 2 block Jacobi; one that stalls is dropped on the way), [5] length of the real
  * vector iterated on, [6] 1 when iterations ran with their vector work
  * carried by the operator launches (FP64 packed solve; with block Jacobi a
  * fusable apply form; fusion on: heomq_ctx_set_precond_fusion; the same
